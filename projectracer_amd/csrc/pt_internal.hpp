@@ -71,15 +71,21 @@ struct VisSet {
   double *vis, *vx, *vz, *vxx, *vzz, *vxz, *vxxpzz, *vxxmzz, *vsmooth;
 };
 
+// a level's RKC1 sweep: core tile, stages per launch, rows per thread
+struct SweepPlan {
+  int cw, ch, ns, rb;
+};
+
 struct Level {
   LevelGeom g;
-  double *err, *bufB, *bufC;      // psi correction and RKC rotating buffers
+  double *err, *bufB, *bufC, *bufD, *bufE;   // psi correction and RKC rotating buffers
   double *rhs, *res, *dts, *ratio;
   double *vis_static;
   VisSet v, vs;                   // primary / scratch viscosity sets
   // FP32 mirrors for the mixed-precision smoother
-  float *ferr, *fB, *fC, *fD, *fE, *frhs, *fdts, *fvis, *fvxm, *fvxz, *fvx, *fvz;
+  float *ferr, *fB, *fC, *fD, *fE, *fres, *frhs, *fdts, *fvis, *fvxm, *fvxz, *fvx, *fvz;
   size_t nelem;                   // (n+7)*(m+7)
+  SweepPlan plan[2];              // tiling of the level's RKC1 sweeps: FP64, FP32
 };
 
 struct KTimer {

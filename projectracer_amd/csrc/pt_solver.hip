@@ -1,9 +1,10 @@
 // pt_solver.hip -- stream-function multigrid on gfx950.
 //
 // Kernels (one HIP kernel per reference loop nest or fused group):
-//   k_stage<R>      fused stream_derivatives + stream_space + RKC1 stage update
-//                   + enforceBCs_stream (ghost write-through), LDS tile with a
-//                   3-wide halo       (PS/iterative_solver.f90:973-1018, 890-911,
+//   k_sweep<R>      several RKC1 stages per launch on LDS tiles: stream_derivatives
+//                   + stream_space + stage update + enforceBCs_stream (ghost
+//                   write-through), and the residual after the last one
+//                                     (PS/iterative_solver.f90:973-1018, 890-911,
 //                                      1561-1597, 1616-1664)
 //   k_residual<R>   stream_derivatives + compute_residual with per-block |r| sums
 //                                      (PS/iterative_solver.f90:415-448)
@@ -16,9 +17,6 @@
 //                   wavefront, and the solve (DGBTRS) as a dense interior operator
 //                   built once per factorization (PS/iterative_solver.f90:1701-1887),
 //                   applied by k_coarse_apply (FP64) or k_coarse_apply_wg (mixed)
-//   k_smooth_small, k_smooth_cb, k_strip_cb
-//                   whole RKC1 sweeps of coarse levels in LDS (one workgroup, or
-//                   column strips with several fused stages per launch)
 //   k_velocities    compute_velocities + velocityBCs (PS/momentum.f90:655-710,
 //                   PS/composition.f90:1295-1325)
 // FP64 kernels are compiled without FMA contraction so each point is
@@ -26,6 +24,7 @@
 #include <cmath>
 #include <cstring>
 #include <algorithm>
+#include <type_traits>
 #include <vector>
 #include "pt_internal.hpp"
 
@@ -36,21 +35,10 @@ namespace pt {
 // ---------------------------------------------------------------------------
 // stencil evaluation of stream_space on an LDS tile
 // ---------------------------------------------------------------------------
-struct Coef {
-  const void *vis, *vxm, *vxz, *vx, *vz, *rhs, *dts;
-};
-
 template <typename R>
 struct StageArgs {
-  const R* Sx;      // stencil input
-  const R* S0;      // pointwise
-  const R* S2;      // pointwise
-  R* Y;             // output (+ mirrored ghosts)
+  const R* Sx;      // the field the operator is applied to
   const R *vis, *vxm, *vxz, *vx, *vz, *rhs, *dts;
-  R c0, c1, c2, cf; // Y = ((c0*S0 + c1*S1) + c2*S2) + ((cf*dt)*F)   (stage >= 2)
-  int stage1;       // Y = S0 + (cf*dt)*F
-  int s0zero;       // S0 == 0 (mixed-precision correction from zero)
-  int ivis0;
   int n, m, pitch;
   R sz;             // ghost sign in z (free-slip -1, rigid +1)
   R dr2, dr3, dr4, ds2, ds3, ds4, drds, dr2ds, drds2, dr2ds2;
@@ -70,6 +58,7 @@ __device__ __forceinline__ float scale_(float s, float d, float rd) { (void)d; r
 
 constexpr int TX = 64, TZ = 8, PZ = 1;
 constexpr size_t SMALL_LDS_BYTES = 160 * 1024;
+constexpr size_t SWEEP_LDS_BYTES = SMALL_LDS_BYTES - 4096;   // two iterates, beside k_sweep's static arrays
 constexpr int TW = TX + 6, TH = TZ * PZ + 6;
 constexpr int TILE_PER = (TH * TW + TX * TZ - 1) / (TX * TZ);   // tile elements per thread
 
@@ -206,46 +195,6 @@ __device__ __forceinline__ void store_with_ghosts(R* Y, int i, int k, int n, int
   }
 }
 
-// one RKC1 stage on a TX x (TZ*PZ) tile; the pointwise operands are loaded
-// before the tile barrier so their latency overlaps the tile fill
-template <typename R, bool IV0>
-__global__ void __launch_bounds__(TX* TZ) k_stage(StageArgs<R> a) {
-  __shared__ R tile[TH][TW];
-  const int i0 = 1 + blockIdx.x * TX, k0 = 1 + blockIdx.y * TZ * PZ;
-  const TileRegs<R> tr = tile_issue<R>(a.Sx, i0, k0, a.n, a.m, a.pitch);
-  R dt[PZ], s0[PZ], s2[PZ];
-  PointCoef<R> pc[PZ];
-  const int i = i0 + threadIdx.x;
-#pragma unroll
-  for (int pz = 0; pz < PZ; pz++) {
-    int k = k0 + threadIdx.y + pz * TZ;
-    dt[pz] = s0[pz] = s2[pz] = (R)0;
-    if (i > a.n - 1 || k > a.m - 1) continue;
-    long g = IDX(i, k, a.pitch);
-    dt[pz] = a.dts[g];
-    if (!a.s0zero) s0[pz] = a.S0[g];
-    if (!a.stage1) s2[pz] = a.S2[g];
-    pc[pz] = load_pc<R, IV0>(a, g);
-  }
-  tile_commit<R>(tile, tr);
-  __syncthreads();
-#pragma unroll
-  for (int pz = 0; pz < PZ; pz++) {
-    int k = k0 + threadIdx.y + pz * TZ;
-    if (i > a.n - 1 || k > a.m - 1) continue;
-    int ti = threadIdx.x + 3, tk = threadIdx.y + pz * TZ + 3;
-    R F = stream_space_pt<R, IV0>([&](int b, int q) { return tile[tk + b][ti + q]; }, a, pc[pz]);
-    R y;
-    if (a.stage1) {
-      y = s0[pz] + (a.cf * dt[pz]) * F;
-    } else {
-      R s1 = tile[tk][ti];
-      y = ((a.c0 * s0[pz] + a.c1 * s1) + a.c2 * s2[pz]) + ((a.cf * dt[pz]) * F);
-    }
-    store_with_ghosts<R>(a.Y, i, k, a.n, a.m, a.pitch, y, a.sz);
-  }
-}
-
 // residual(i,k) = stream_space(i,k,S); block partial sums of |residual|
 template <typename R, bool IV0>
 __global__ void __launch_bounds__(TX* TZ) k_residual(StageArgs<R> a, R* res, double* partial) {
@@ -305,15 +254,6 @@ __global__ void k_rk1_update(double* psi, const double* F, const double* dts, co
   store_with_ghosts<double>(psi, i, k, n, m, pitch, y, sz);
 }
 
-// ---------------------------------------------------------------------------
-// small levels: the whole RKC1 sweep (all stages) and compute_residual in one
-// workgroup with the three RKC buffers resident in LDS.  Each thread owns up
-// to PPT interior points; their indices and pointwise operands are fixed for
-// the sweep and kept in registers.
-// ---------------------------------------------------------------------------
-struct RkcCoef {
-  double mewt[64], mew[64], vv[64], cc[64];
-};
 // the RKC1 stage count and coefficients of a level's sweeps: the reference's
 // nstageS everywhere, or s_coarse stages on the mixed path's levels >= 2
 struct LevelRkc {
@@ -326,433 +266,330 @@ static LevelRkc level_rkc(const Context& c, int l, bool fp32) {
   if (fp32 && l >= 2 && t.s_coarse >= 2) return {t.s_coarse, t.mewt_c, t.mew_c, t.vv_c, t.cc_c, t.RKC1_stability_c};
   return {c.P.nstageS, t.mewt, t.mew, t.vv, t.cc, t.RKC1_stability};
 }
-static RkcCoef rkc_coef(const LevelRkc& rk) {
-  RkcCoef co;
-  std::memcpy(co.mewt, rk.mewt, sizeof co.mewt); std::memcpy(co.mew, rk.mew, sizeof co.mew);
-  std::memcpy(co.vv, rk.vv, sizeof co.vv); std::memcpy(co.cc, rk.cc, sizeof co.cc);
-  return co;
-}
-// the FP32 sweep's stage coefficients, rounded once on the host: c0 = cc,
-// c1 = mew, c2 = vv, cf = mewt * cpar (the product in FP64, as the device
-// would form it); read at a uniform stage index they are scalar loads of
-// the kernel arguments
-struct RkcCoefF {
-  float c0[64], c1[64], c2[64], cf[64];
-};
-static RkcCoefF rkc_f32(const RkcCoef& co, double cpar) {
-  RkcCoefF f;
-  for (int j = 0; j < 64; j++) {
-    f.c0[j] = (float)co.cc[j];
-    f.c1[j] = (float)co.mew[j];
-    f.c2[j] = (float)co.vv[j];
-    f.cf[j] = (float)(co.mewt[j] * cpar);
-  }
-  return f;
-}
 constexpr int SMALL_THREADS = 1024;
 
-// RKC1 coefficients of stages 0..63 held one stage per lane of every
-// wavefront, read at a (uniform) stage index with v_readlane: no memory
-// access in the stage loop
-struct LaneRkc {
-  double cc, mew, vv, mewt;
-};
-__device__ __forceinline__ LaneRkc lane_rkc(const RkcCoef& co) {
-  const int j = threadIdx.x & 63;
-  return LaneRkc{co.cc[j], co.mew[j], co.vv[j], co.mewt[j]};
-}
-__device__ __forceinline__ double lane_at(double v, int j) {
-  const int lo = __builtin_amdgcn_readlane(__double2loint(v), j);
-  const int hi = __builtin_amdgcn_readlane(__double2hiint(v), j);
-  return __hiloint2double(hi, lo);
-}
+// ---------------------------------------------------------------------------
+// RKC1 sweeps, several stages per launch.  A workgroup owns a core tile of a
+// level and computes `ns` consecutive stages on it: the current iterate S1 is
+// in LDS (two buffers, one barrier per stage) on the core widened by 3 points
+// per evaluation, every point's S0, S2, dt_stream, RHS and viscosity
+// coefficients stay in the registers of the thread that owns it, and stage t
+// is evaluated on the core widened by 3 points per evaluation still to come,
+// so tiles do not exchange anything within a launch (overlap points are
+// computed by both neighbours).  A tile that covers the whole level takes the
+// whole sweep in one launch.  Each thread owns RB vertically adjacent points
+// of one column and reads their common neighbourhood once.  Per point the
+// operations and their order are those of one stage per launch
+// (stream_space_pt, or the factorised form below), so the results do not
+// depend on the tiling.
+// ---------------------------------------------------------------------------
+constexpr int SWEEP_MAX_STAGES = 64;
 
-// a level array into LDS (and two more LDS arrays zeroed) by a whole
-// workgroup of NT threads, B elements per thread per batch: the batch's
-// loads (indices clamped into the array) are all issued before its first
-// LDS write
-template <typename R, int NT, int B>
-__device__ __forceinline__ void copy_in3(const R* src, R* d0, R* d1, R* d2, int ne) {
-  for (int e0 = threadIdx.x; e0 < ne; e0 += B * NT) {
-    R v[B];
+// the distinct stencil weights: D1 and D3 are odd, D2 and D4 even, and the
+// mixed ones are their products, so the signs are known at compile time and
+// the 31 magnitudes stay in scalar registers
+template <typename R>
+struct SweepWeights {
+  R d2[3], d3[3], d4[4];       // d3: offsets -1, -2, -3
+  R rs[3], rrs[6], rss[6], rrss[6];
+};
+
+template <typename R>
+struct SweepArgs {
+  const R* S0;      // sweep start (pointwise; stencil source of stage 1)
+  const R* Gcur;    // stage j0-1 (S0 when j0 = 1)
+  const R* Gprev;   // stage j0-2 (an allocated level buffer also when j0 = 1)
+  R* Ocur;          // the last stage on the core, with ghost images
+  R* Oprev;         // the stage before it; null on the sweep's last launch
+  R* res;           // RHS - L psi of the last stage on the core; null: not wanted
+  const R *vis, *vxm, *vxz, *vx, *vz, *rhs, *dts;
+  int n, m, pitch;
+  int j0, ns;       // first stage (1-based) and number of stages
+  int cw, ch, nbx;  // core size, tiles per row
+  int w1, nrb, tcol;  // columns of the first stage's region, its blocks of RB rows, threads per block row
+  R sz;
+  R dr2, dr3, dr4, ds2, ds3, ds4, drds, dr2ds, drds2, dr2ds2;
+  R rdr2, rdr3, rdr4, rds2, rds3, rds4, rdrds, rdr2ds, rdrds2, rdr2ds2;
+  SweepWeights<R> w;
+  R c0[SWEEP_MAX_STAGES], c1[SWEEP_MAX_STAGES], c2[SWEEP_MAX_STAGES], cf[SWEEP_MAX_STAGES];
+};
+
+// s / d, correctly rounded, from rd = RN(1/d).  PW2: d is a power of two and
+// the product is the quotient.  Otherwise two residual corrections: the first
+// leaves q within one unit of the quotient, and then the second rounds it
+// correctly (Markstein's theorem).  A quotient that overflows is returned as
+// it is (the correction of an infinity would be NaN).
+template <bool PW2>
+__device__ __forceinline__ double quot(double s, double d, double rd) {
+  const double q0 = s * rd;
+  if constexpr (PW2) return q0;
+  const double q1 = __fma_rn(__fma_rn(-q0, d, s), rd, q0);
+  const double q2 = __fma_rn(__fma_rn(-q1, d, s), rd, q1);
+  return fabs(q0) < INFINITY ? q2 : q0;
+}
+template <bool PW2>
+__device__ __forceinline__ float quot(float s, float d, float rd) { (void)d; return s * rd; }
+
+// Sums of the derivatives at one point, updated row by row: row(b, e, x) adds
+// the row b points above the point (e: its five values around the column;
+// x: on the point's own row the values 3 columns away).  Called with b = -3
+// .. 3 in order, every sum is accumulated in stream_space_pt's order.
+// EV 0: general operator; 1: isoviscous; 2: isoviscous with psi_xxzz as
+// D2_z(D2_x psi) (FP32 levels >= 2)
+template <typename R, int EV>
+struct PointSums {
+  R sxx, szz, sxxx, szzz, sxxxx, szzzz, sxz, sxxz, sxzz, sxxzz;
+  __device__ __forceinline__ void clear() {
+    sxx = szz = sxxx = szzz = sxxxx = szzzz = sxz = sxxz = sxzz = sxxzz = (R)0;
+  }
+  template <int B>
+  __device__ __forceinline__ void row(const SweepWeights<R>& w, const R* e, R xl, R xr, R d2x) {
+    constexpr int ab = B < 0 ? -B : B;
+    if constexpr (B == 0) {
+      const R at[7] = {xl, e[0], e[1], e[2], e[3], e[4], xr};
+      if constexpr (EV == 0) {
 #pragma unroll
-    for (int u = 0; u < B; u++) v[u] = src[min(e0 + u * NT, ne - 1)];
+        for (int q = -2; q <= 2; q++) sxx = acc_(sxx, w.d2[abs(q)], at[q + 3]);
 #pragma unroll
-    for (int u = 0; u < B; u++) {
-      const int e = e0 + u * NT;
-      if (e < ne) {
-        d0[e] = v[u];
-        d1[e] = (R)0;
-        d2[e] = (R)0;
+        for (int q = -3; q <= 3; q++) if (q != 0) sxxx = acc_(sxxx, q < 0 ? w.d3[-q - 1] : -w.d3[q - 1], at[q + 3]);
+      }
+      if constexpr (EV == 2) sxxxx = w.d4[3] * xl;
+      else sxxxx = acc_(sxxxx, w.d4[3], xl);
+#pragma unroll
+      for (int q = -2; q <= 3; q++) sxxxx = acc_(sxxxx, w.d4[abs(q)], at[q + 3]);
+    }
+    if constexpr (EV == 0) {
+      if constexpr (ab <= 2) szz = acc_(szz, w.d2[ab], e[2]);
+      if constexpr (B != 0) szzz = acc_(szzz, B < 0 ? w.d3[ab - 1] : -w.d3[ab - 1], e[2]);
+    }
+    szzzz = acc_(szzzz, w.d4[ab], e[2]);
+    if constexpr (ab <= 2 && EV == 2) sxxzz = acc_(sxxzz, w.d2[ab], d2x);
+    if constexpr (ab <= 2 && EV != 2) {
+#pragma unroll
+      for (int q = -2; q <= 2; q++) {
+        const R v = e[q + 2];
+        const int aq = abs(q);
+        if constexpr (EV == 0) {
+          // D1 is odd: negative where exactly one offset is
+          if (B != 0 && q != 0) sxz = acc_(sxz, (B < 0) != (q < 0) ? -w.rs[ab + aq - 2] : w.rs[ab + aq - 2], v);
+          if (B != 0) sxxz = acc_(sxxz, B < 0 ? w.rrs[(ab - 1) * 3 + aq] : -w.rrs[(ab - 1) * 3 + aq], v);
+          if (q != 0) sxzz = acc_(sxzz, q < 0 ? w.rss[(aq - 1) * 3 + ab] : -w.rss[(aq - 1) * 3 + ab], v);
+        }
+        const int lo = ab < aq ? ab : aq, hi = ab < aq ? aq : ab;
+        sxxzz = acc_(sxxzz, w.rrss[lo == 0 ? hi : lo == 1 ? 2 + hi : 5], v);
       }
     }
   }
-}
-
-template <typename R, bool IV0, int PPT>
-__device__ __forceinline__ void sweep_small(const StageArgs<R>& a, R* err, R* res, int nstage, double cpar,
-                                            const RkcCoef& co, R* buf0) {
-  const int n = a.n, m = a.m, p = a.pitch;
-  const int ne = p * (m + 7);
-  R* buf1 = buf0 + ne;
-  R* buf2 = buf1 + ne;
-  const int tid = threadIdx.x;
-  copy_in3<R, SMALL_THREADS, 8>(err, buf0, buf1, buf2, ne);
-  // point e of the thread's PPT: row e / tcol, column e % tcol, with rows
-  // of tcol points padded to whole wavefronts when the workgroup has room,
-  // so that no wave spans two rows (lanes a row lower hit other lanes' LDS
-  // banks)
-  const int nxi = n - 1;
-  const int padded = (nxi + 63) & ~63;
-  const int tcol = padded * (m - 1) <= PPT * SMALL_THREADS ? padded : nxi;
-  const int npts = tcol * (m - 1);
-  int pi[PPT], pk[PPT], pg[PPT];
-  R pdt[PPT];
-  PointCoef<R> pc[PPT];
-#pragma unroll
-  for (int q = 0; q < PPT; q++) {
-    int e = tid + q * SMALL_THREADS;
-    pi[q] = 0;
-    pk[q] = 0;
-    pg[q] = 0;
-    pdt[q] = (R)0;
-    const int k = e / tcol, ic = e - k * tcol;
-    if (e < npts && ic < nxi) {
-      pi[q] = 1 + ic;
-      pk[q] = 1 + k;
-      pg[q] = (int)IDX(pi[q], pk[q], p);
-      pdt[q] = a.dts[pg[q]];
-      pc[q] = load_pc<R, IV0>(a, pg[q]);
+  // RHS - L psi from the sums (stream_space)
+  template <bool PW2>
+  __device__ __forceinline__ R value(const SweepArgs<R>& a, const PointCoef<R>& pc) const {
+    if constexpr (EV == 2) {
+      const R lap2 = sxxxx * a.rdr4 + szzzz * a.rds4 + (R)2 * (sxxzz * a.rdr2ds2);
+      return pc.rhs - pc.vis * lap2;
+    } else {
+      const R SFxxxx = quot<PW2>(sxxxx, a.dr4, a.rdr4), SFzzzz = quot<PW2>(szzzz, a.ds4, a.rds4);
+      const R SFxxzz = quot<PW2>(sxxzz, a.dr2ds2, a.rdr2ds2);
+      const R t2 = pc.vis * (SFxxxx + SFzzzz + (R)2 * SFxxzz);
+      if constexpr (EV == 1) return -(t2 - pc.rhs);
+      const R SFxx = quot<PW2>(sxx, a.dr2, a.rdr2), SFxxx = quot<PW2>(sxxx, a.dr3, a.rdr3);
+      const R SFzz = quot<PW2>(szz, a.ds2, a.rds2), SFzzz = quot<PW2>(szzz, a.ds3, a.rds3);
+      const R SFxz = quot<PW2>(sxz, a.drds, a.rdrds), SFxxz = quot<PW2>(sxxz, a.dr2ds, a.rdr2ds);
+      const R SFxzz = quot<PW2>(sxzz, a.drds2, a.rdrds2);
+      const R t1 = pc.vxm * (SFxx - SFzz);
+      const R t4 = ((R)4 * pc.vxz) * SFxz;
+      const R t5 = ((R)2 * pc.vx) * (SFxxx + SFxzz);
+      const R t6 = ((R)2 * pc.vz) * (SFzzz + SFxxz);
+      return -(t1 + t2 + t4 + t5 + t6 - pc.rhs);
     }
   }
-  const LaneRkc lk = lane_rkc(co);
-  __syncthreads();
-  // stage 1: S1 = S0 + mewt1*c*dt*F(S0) -> buf1
-  {
-    const R cf = (R)(lane_at(lk.mewt, 1) * cpar);
-#pragma unroll
-    for (int q = 0; q < PPT; q++) {
-      if (pi[q] == 0) continue;
-      const int g = pg[q];
-      R F = stream_space_pt<R, IV0>([&](int b, int c) { return buf0[g + b * p + c]; }, a, pc[q]);
-      R y = buf0[g] + (cf * pdt[q]) * F;
-      store_with_ghosts<R>(buf1, pi[q], pk[q], n, m, p, y, a.sz);
-    }
-  }
-  __syncthreads();
-  R* cur = buf1;
-  R* prev = buf0;   // S2 = S0 at stage 2
-  R* spare = buf2;
-  for (int j = 2; j <= nstage; j++) {
-    R* out = (prev == buf0) ? spare : prev;
-    const R c0 = (R)lane_at(lk.cc, j), c1 = (R)lane_at(lk.mew, j), c2 = (R)lane_at(lk.vv, j);
-    const R cf = (R)(lane_at(lk.mewt, j) * cpar);
-#pragma unroll
-    for (int q = 0; q < PPT; q++) {
-      if (pi[q] == 0) continue;
-      const int g = pg[q];
-      R F = stream_space_pt<R, IV0>([&](int b, int c) { return cur[g + b * p + c]; }, a, pc[q]);
-      R y = ((c0 * buf0[g] + c1 * cur[g]) + c2 * prev[g]) + ((cf * pdt[q]) * F);
-      store_with_ghosts<R>(out, pi[q], pk[q], n, m, p, y, a.sz);
-    }
-    __syncthreads();
-    R* np = cur;
-    cur = out;
-    prev = np;
-    if (out == spare) spare = nullptr;
-  }
-  // cur holds the sweep result (psi correction): write back, then the residual
-  for (int e = tid; e < ne; e += SMALL_THREADS) err[e] = cur[e];
-#pragma unroll
-  for (int q = 0; q < PPT; q++) {
-    if (pi[q] == 0) continue;
-    const int g = pg[q];
-    res[g] = stream_space_pt<R, IV0>([&](int b, int c) { return cur[g + b * p + c]; }, a, pc[q]);
-  }
-}
-
-template <typename R, bool IV0, int PPT>
-__global__ void __launch_bounds__(SMALL_THREADS) k_smooth_small(StageArgs<R> a, R* err, R* res, int nstage,
-                                                               double cpar, RkcCoef co) {
-  extern __shared__ unsigned char smem_raw[];
-  sweep_small<R, IV0, PPT>(a, err, res, nstage, cpar, co, reinterpret_cast<R*>(smem_raw));
-}
-
-// F = RHS - L psi (isoviscous, FP32) at the RB vertically adjacent points
-// (i, k0..k0+RB-1) of an LDS array with row pitch W whose column 0 is global
-// column `lo` and whose row 0 is global row -3.  The x-D2 sums of the RB+4
-// rows the 5x5 neighbourhood spans are formed once and reused by every
-// point's z-D2 sum (psi_xxzz = D2_z(D2_x psi), the product weights D2(b)D2(q)
-// factorised); each LDS value is read once.  Rows beyond rmax (points past
-// the last interior row of a partial block) are clamped; their F is unused.
-template <int RB>
-__device__ __forceinline__ void eval_cb(const float* S, int W, int lo, int i, int k0, int rmax,
-                                        const StageArgs<float>& a, const float* rhsv, const float* visv, float* F) {
-  auto at = [&](int ii, int kk) { return S[(kk + 3) * W + (ii - lo)]; };
-  float v[5][RB + 4];
-#pragma unroll
-  for (int w = 0; w < RB + 4; w++) {
-    const int row = min(k0 - 2 + w, rmax);
-#pragma unroll
-    for (int c = 0; c < 5; c++) v[c][w] = at(i - 2 + c, row);
-  }
-  float colv[RB + 6];
-  colv[0] = at(i, k0 - 3);
-#pragma unroll
-  for (int w = 0; w < RB + 4; w++) colv[w + 1] = v[2][w];
-  colv[RB + 5] = at(i, min(k0 + RB + 2, rmax));
-  float t2[RB + 4];
-#pragma unroll
-  for (int w = 0; w < RB + 4; w++) {
-    float acc = 0.0f;
-#pragma unroll
-    for (int c = 0; c < 5; c++) acc = __fmaf_rn(a.D2[c], v[c][w], acc);
-    t2[w] = acc;
-  }
-#pragma unroll
-  for (int r = 0; r < RB; r++) {
-    const int w = r + 2;
-    const int row = min(k0 + r, rmax);
-    float sxxxx = a.D4[0] * at(i - 3, row);
-#pragma unroll
-    for (int c = 0; c < 5; c++) sxxxx = __fmaf_rn(a.D4[c + 1], v[c][w], sxxxx);
-    sxxxx = __fmaf_rn(a.D4[6], at(i + 3, row), sxxxx);
-    float szzzz = 0.0f;
-#pragma unroll
-    for (int b = 0; b < 7; b++) szzzz = __fmaf_rn(a.D4[b], colv[r + b], szzzz);
-    float sxxzz = 0.0f;
-#pragma unroll
-    for (int b = 0; b < 5; b++) sxxzz = __fmaf_rn(a.D2[b], t2[w - 2 + b], sxxzz);
-    const float lap2 = sxxxx * a.rdr4 + szzzz * a.rds4 + 2.0f * (sxxzz * a.rdr2ds2);
-    F[r] = rhsv[r] - visv[r] * lap2;
-  }
-}
-
-// FP32 isoviscous single-workgroup sweep for the mixed-precision smoother,
-// column-blocked: each thread owns RB vertically adjacent points of one
-// column (eval_cb); S0 and the pointwise operands stay in registers.
-// Factorised sums round differently from the reference's 5x5 product
-// weights, so only the FP32 path uses this.
-template <int RB>
-__device__ __forceinline__ void sweep_cb(const StageArgs<float>& a, float* err, float* res, int nstage,
-                                         const RkcCoefF& co, float* buf0) {
-  const int n = a.n, m = a.m, p = a.pitch;
-  const int ne = p * (m + 7);
-  float* buf1 = buf0 + ne;
-  float* buf2 = buf1 + ne;
-  const int tid = threadIdx.x;
-  // threads of a row block: the n-1 interior columns, padded to whole
-  // wavefronts when the workgroup has room, so that no wave spans two row
-  // blocks (lanes one block lower hit other lanes' LDS banks)
-  const int nxi = n - 1, nkb = (m - 1 + RB - 1) / RB;
-  const int padded = (nxi + 63) & ~63;
-  const int tcol = padded * nkb <= SMALL_THREADS ? padded : nxi;
-  const int kb = tid / tcol, ic = tid - kb * tcol;
-  const bool active = kb < nkb && ic < nxi;
-  int i = 1, k0 = 1;
-  float s0v[RB], dtv[RB], rhsv[RB], visv[RB];
-  bool on[RB];
-  if (active) {
-    i = 1 + ic;
-    k0 = 1 + kb * RB;
-  }
-  // the pointwise operands from clamped (valid) points, zero where the
-  // thread has no point; issued before the copy-in so that both are in
-  // flight together
-#pragma unroll
-  for (int r = 0; r < RB; r++) {
-    int k = k0 + r;
-    on[r] = active && k <= m - 1;
-    const long g = IDX(i, min(k, m - 1), p);
-    const float e0 = err[g], d0 = a.dts[g], r0 = a.rhs[g], v0 = a.vis[g];
-    s0v[r] = on[r] ? e0 : 0.0f;
-    dtv[r] = on[r] ? d0 : 0.0f;
-    rhsv[r] = on[r] ? r0 : 0.0f;
-    visv[r] = on[r] ? v0 : 0.0f;
-  }
-  copy_in3<float, SMALL_THREADS, 8>(err, buf0, buf1, buf2, ne);
-  const int rmax = m + 3;   // last stored row
-  __syncthreads();
-  {
-    const float cf = co.cf[1];
-    float F[RB];
-    eval_cb<RB>(buf0, p, -3, i, k0, rmax, a, rhsv, visv, F);
-#pragma unroll
-    for (int r = 0; r < RB; r++)
-      if (on[r]) store_with_ghosts<float>(buf1, i, k0 + r, n, m, p, s0v[r] + (cf * dtv[r]) * F[r], a.sz);
-  }
-  __syncthreads();
-  float* cur = buf1;
-  float* prev = buf0;   // S2 = S0 at stage 2
-  float* spare = buf2;
-  for (int j = 2; j <= nstage; j++) {
-    float* out = (prev == buf0) ? spare : prev;
-    const float c0 = co.c0[j], c1 = co.c1[j], c2 = co.c2[j], cf = co.cf[j];
-    float F[RB];
-    eval_cb<RB>(cur, p, -3, i, k0, rmax, a, rhsv, visv, F);
-#pragma unroll
-    for (int r = 0; r < RB; r++) {
-      if (!on[r]) continue;
-      long g = IDX(i, k0 + r, p);
-      float y = ((c0 * s0v[r] + c1 * cur[g]) + c2 * prev[g]) + ((cf * dtv[r]) * F[r]);
-      store_with_ghosts<float>(out, i, k0 + r, n, m, p, y, a.sz);
-    }
-    __syncthreads();
-    float* np = cur;
-    cur = out;
-    prev = np;
-    if (out == spare) spare = nullptr;
-  }
-  for (int e = tid; e < ne; e += SMALL_THREADS) err[e] = cur[e];
-  float F[RB];
-  eval_cb<RB>(cur, p, -3, i, k0, rmax, a, rhsv, visv, F);
-#pragma unroll
-  for (int r = 0; r < RB; r++)
-    if (on[r]) res[IDX(i, k0 + r, p)] = F[r];
-}
-
-template <int RB>
-__global__ void __launch_bounds__(SMALL_THREADS) k_smooth_cb(StageArgs<float> a, float* err, float* res, int nstage,
-                                                            RkcCoefF co) {
-  extern __shared__ unsigned char smem_raw[];
-  sweep_cb<RB>(a, err, res, nstage, co, reinterpret_cast<float*>(smem_raw));
-}
-
-// ---------------------------------------------------------------------------
-// FP32 isoviscous RKC1 sweep segments on column strips (temporal blocking),
-// for levels too large for one workgroup.  Workgroup b owns the core columns
-// [c0, c1) and keeps whole columns (rows -3..m+3) of the core widened by 3
-// columns per fused stage in LDS.  Stage t of a segment is computed on the
-// core widened by 3 columns per remaining stage, so after the segment the
-// core holds its last stage with no exchange between workgroups (overlap
-// columns are computed by both neighbours).  Per point the arithmetic is
-// eval_cb's, so the result does not depend on the strip decomposition.
-// Threads: x = strip column (64 lanes), y = 16 blocks of 4 rows (m <= 65).
-// ---------------------------------------------------------------------------
-constexpr int STRIP_TX = 64, STRIP_TY = 16, STRIP_RB = 4;
-
-struct StripArgs {
-  const float* S0;    // sweep start (pointwise; stencil source of stage 1)
-  const float* Gcur;  // stage j0-1, read when j0 >= 3
-  const float* Gprev; // stage j0-2, used when j0 >= 3 (an allocated level buffer: always loaded)
-  float* Ocur;        // stage j1 on the core columns (+ ghost images)
-  float* Oprev;       // stage j1-1 on the core columns; null on the last segment
-  int j0, j1;         // stages of this segment (1-based, j1 > j0)
-  int cw;             // core columns per workgroup
-  int W;              // LDS strip width in columns
-  RkcCoefF co;        // stage coefficients, cf with the sweep's Courant factor
 };
 
-__global__ void __launch_bounds__(STRIP_TX* STRIP_TY) k_strip_cb(StageArgs<float> a, StripArgs s) {
+// rows ROW .. RB+2 around a thread's RB points (S: the first point's place in
+// LDS), each read once and added to every point it belongs to; s1 receives
+// the points' own values, and a point's F = RHS - L psi is formed as soon as
+// its last row is in, so that few sums and rows are live at a time
+template <typename R, int EV, int RB, bool PW2, int ROW>
+__device__ __forceinline__ void sweep_rows(const R* S, int W, const SweepArgs<R>& a, const PointCoef<R>* pc,
+                                           PointSums<R, EV>* ps, R* s1, R* F) {
+  if constexpr (ROW <= RB + 2) {
+    constexpr bool five = ROW >= -2 && ROW <= RB + 1, own = ROW >= 0 && ROW < RB;
+    R e[5], xl = 0, xr = 0, d2x = 0;
+    const R* q = S + ROW * W;
+    e[2] = q[0];
+    if constexpr (five) { e[0] = q[-2]; e[1] = q[-1]; e[3] = q[1]; e[4] = q[2]; }
+    if constexpr (own) { xl = q[-3]; xr = q[3]; s1[ROW] = e[2]; }
+    if constexpr (EV == 2 && five) {
+#pragma unroll
+      for (int c = 0; c < 5; c++) d2x = acc_(d2x, a.w.d2[abs(c - 2)], e[c]);
+    }
+    auto add = [&](auto rc) {
+      constexpr int r = decltype(rc)::value, B = ROW - r;
+      if constexpr (r < RB && B >= -3 && B <= 3) {
+        if constexpr (B == -3) ps[r].clear();
+        ps[r].template row<B>(a.w, e, xl, xr, d2x);
+        if constexpr (B == 3) F[r] = ps[r].template value<PW2>(a, pc[r]);
+      }
+    };
+    add(std::integral_constant<int, 0>{});
+    add(std::integral_constant<int, 1>{});
+    add(std::integral_constant<int, 2>{});
+    add(std::integral_constant<int, 3>{});
+    sweep_rows<R, EV, RB, PW2, ROW + 1>(S, W, a, pc, ps, s1, F);
+  }
+}
+
+template <typename R, int EV, int RB, int NT, bool PW2>
+__global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT / 256, NT / 256))) k_sweep(SweepArgs<R> a) {
+  static_assert(RB <= 4, "sweep_rows handles up to 4 points per thread");
   extern __shared__ unsigned char smem_raw[];
-  constexpr int RB = STRIP_RB;
-  const int n = a.n, m = a.m, p = a.pitch;
-  const int halo = 3 * (s.j1 - s.j0 + 1);
-  const int c0 = 1 + blockIdx.x * s.cw, c1 = min(c0 + s.cw, n);   // core [c0, c1)
-  const int lo = max(-3, c0 - halo), hi = min(n + 3, c1 - 1 + halo);
-  const int W = s.W, rows = m + 7;
-  float* const buf = reinterpret_cast<float*>(smem_raw);   // three strips of W*rows
-  const int bsz = W * rows;
-  const int tid = threadIdx.y * STRIP_TX + threadIdx.x, nthr = STRIP_TX * STRIP_TY;
-  const float* cur_src = (s.j0 == 1) ? s.S0 : s.Gcur;
-  const bool has_prev = s.j0 >= 3;
-  // this thread's column and row block; pointwise operands in registers,
-  // loaded from clamped (valid) points and zero where the thread has none
-  const int ic = c0 - halo + 3 + threadIdx.x;
-  const int k0 = 1 + threadIdx.y * RB;
-  float s0v[RB], dtv[RB], rhsv[RB], visv[RB];
-  bool on[RB];
+  const int n = a.n, m = a.m, p = a.pitch, ns = a.ns;
+  const int nev = ns + (a.res ? 1 : 0);   // evaluations of the operator
+  const int bx = blockIdx.x % a.nbx, bz = blockIdx.x / a.nbx;
+  const int cx0 = 1 + bx * a.cw, cx1 = min(cx0 + a.cw, n);   // core [cx0, cx1) x [cz0, cz1)
+  const int cz0 = 1 + bz * a.ch, cz1 = min(cz0 + a.ch, m);
+  // LDS window: the first evaluation's region and 3 points around it (4
+  // where it starts at a wall), rows padded to whole blocks of RB
+  const int x1 = max(1, cx0 - 3 * (nev - 1)), z1 = max(1, cz0 - 3 * (nev - 1));
+  const int ilo = max(-3, cx0 - 3 * nev), klo = max(-3, cz0 - 3 * nev);
+  const int W = a.w1 + 8, rows = a.nrb * RB + 8, ne = W * rows;
+  R* const buf = reinterpret_cast<R*>(smem_raw);
+  const int tid = threadIdx.x, nthr = blockDim.x;
+  __shared__ R coef[4][SWEEP_MAX_STAGES];
+  if (tid < SWEEP_MAX_STAGES) {   // at least one wavefront
+    const int j = min(a.j0 + tid, SWEEP_MAX_STAGES - 1);
+    coef[0][tid] = a.c0[j]; coef[1][tid] = a.c1[j]; coef[2][tid] = a.c2[j]; coef[3][tid] = a.cf[j];
+  }
+  // the window: each batch's loads are issued before its LDS writes
+  constexpr int FB = 4;
+  for (int e0 = tid; e0 < ne; e0 += FB * nthr) {
+    R v[FB];
+#pragma unroll
+    for (int u = 0; u < FB; u++) {
+      const int e = min(e0 + u * nthr, ne - 1);
+      const int rr = e / W, cc = e - rr * W;
+      v[u] = a.Gcur[IDX(min(ilo + cc, n + 3), min(klo + rr, m + 3), p)];
+    }
+#pragma unroll
+    for (int u = 0; u < FB; u++) {
+      const int e = e0 + u * nthr;
+      if (e < ne) {
+        buf[e] = v[u];
+        buf[ne + e] = (R)0;   // the walls' psi = 0 and the ghosts of the other buffer
+      }
+    }
+  }
+  // this thread's column and row block; its points' operands, from clamped
+  // (valid) points
+  const int rb = tid / a.tcol, ic = x1 + (tid - rb * a.tcol);
+  const int k0 = z1 + rb * RB;
+  const bool col = rb < a.nrb && tid - rb * a.tcol < a.w1 && ic <= n - 1;
+  R s0v[RB], pv[RB], yv[RB], dtv[RB];
+  PointCoef<R> pc[RB];
+#pragma unroll
+  for (int r = 0; r < RB; r++) {
+    const long g = IDX(min(ic, n - 1), min(k0 + r, m - 1), p);
+    s0v[r] = a.S0[g];
+    pv[r] = a.Gprev[g];
+    dtv[r] = a.dts[g];
+    pc[r].rhs = a.rhs[g];
+    pc[r].vis = a.vis[g];
+    if constexpr (EV == 0) {
+      pc[r].vxm = a.vxm[g]; pc[r].vxz = a.vxz[g]; pc[r].vx = a.vx[g]; pc[r].vz = a.vz[g];
+    }
+    yv[r] = (R)0;
+  }
+  __syncthreads();
+  int at0 = 0;   // LDS offset of the current iterate
+  const int own = (k0 - klo) * W + (ic - ilo);
+  // LDS offsets of the points' ghost images (antisymmetric side walls,
+  // sz-symmetric top and bottom), 0 where there is none.  On levels of at
+  // least 7 cells a point has at most one image per direction; smaller ones
+  // take the general form
+  const bool tiny = n < 7 || m < 7;
+  int gx = 0, gz[RB];
+  if (ic <= 3 && -ic >= ilo) gx = -2 * ic;
+  else if (ic >= n - 3 && 2 * n - ic < ilo + W) gx = 2 * (n - ic);
 #pragma unroll
   for (int r = 0; r < RB; r++) {
     const int k = k0 + r;
-    on[r] = ic >= 1 && ic <= n - 1 && k <= m - 1;
-    const long g = IDX(min(max(ic, 1), n - 1), min(k, m - 1), p);
-    const float e0 = s.S0[g], d0 = a.dts[g], r0 = a.rhs[g], v0 = a.vis[g];
-    s0v[r] = on[r] ? e0 : 0.0f;
-    dtv[r] = on[r] ? d0 : 0.0f;
-    rhsv[r] = on[r] ? r0 : 0.0f;
-    visv[r] = on[r] ? v0 : 0.0f;
+    gz[r] = 0;
+    if (k <= 3 && -k >= klo) gz[r] = -2 * k * W;
+    else if (k >= m - 3 && 2 * m - k < klo + rows) gz[r] = 2 * (m - k) * W;
   }
-  // the strips: each batch's loads (columns clamped to the strip, both
-  // source buffers always allocated) issued before its LDS writes
-  constexpr int SB = 8;
-  const int nfill = W * rows;
-  for (int e0 = tid; e0 < nfill; e0 += SB * nthr) {
-    float vc[SB], vp[SB];
-#pragma unroll
-    for (int u = 0; u < SB; u++) {
-      const int e = min(e0 + u * nthr, nfill - 1);
-      const int rr = e / W, lc = e - rr * W;
-      const long g = IDX(min(lo + lc, hi), rr - 3, p);
-      vc[u] = cur_src[g];
-      vp[u] = s.Gprev[g];
-    }
-#pragma unroll
-    for (int u = 0; u < SB; u++) {
-      const int e = e0 + u * nthr;
-      if (e < nfill) {
-        const int rr = e / W, lc = e - rr * W;
-        const bool in = lo + lc <= hi;
-        buf[e] = in ? vc[u] : 0.0f;
-        buf[bsz + e] = (in && has_prev) ? vp[u] : 0.0f;
-        buf[2 * bsz + e] = 0.0f;
+  for (int t = 0; t < nev; t++) {
+    const int h = 3 * (nev - 1 - t);
+    if (col && ic >= cx0 - h && ic < cx1 + h && k0 < cz1 + h && k0 + RB > cz0 - h) {
+      // the stage's coefficients: from LDS with the window, or (FP64 general
+      // operator, short of vector registers) scalar
+      R cc0, cc1, cc2, cf;
+      if constexpr (sizeof(R) == 8 && EV == 0) {
+        const int j = a.j0 + t;
+        cc0 = a.c0[j]; cc1 = a.c1[j]; cc2 = a.c2[j]; cf = a.cf[j];
+      } else {
+        cc0 = coef[0][t]; cc1 = coef[1][t]; cc2 = coef[2][t]; cf = coef[3][t];
       }
-    }
-  }
-  const int rmax = m + 3;
-  auto put = [&](float* B, int ii, int kk, float v) {
-    if (ii >= lo && ii <= hi) B[(kk + 3) * W + (ii - lo)] = v;
-  };
-  __syncthreads();
-  int ci = 0, pi = 1;
-  for (int j = s.j0; j <= s.j1; j++) {
-    const int t = j - s.j0;
-    const int rlo = max(1, c0 - halo + 3 * (t + 1)), rhi = min(n - 1, c1 - 1 + halo - 3 * (t + 1));
-    const int oi = 3 - ci - pi;
-    const float* cur = buf + ci * bsz;
-    const float* prev = buf + pi * bsz;
-    float* out = buf + oi * bsz;
-    const float cc0 = s.co.c0[j], cc1 = s.co.c1[j], cc2 = s.co.c2[j], cf = s.co.cf[j];
-    if (ic >= rlo && ic <= rhi && k0 <= m - 1) {
-      float F[RB];
-      eval_cb<RB>(cur, W, lo, ic, k0, rmax, a, rhsv, visv, F);
+      R F[RB], s1[RB];
+      PointSums<R, EV> ps[RB];
+      sweep_rows<R, EV, RB, PW2, -3>(buf + at0 + own, W, a, pc, ps, s1, F);
+      if (t == ns) {
 #pragma unroll
-      for (int r = 0; r < RB; r++) {
-        if (!on[r]) continue;
-        const int k = k0 + r;
-        const int lg = (k + 3) * W + (ic - lo);
-        float y;
-        if (j == 1) y = s0v[r] + (cf * dtv[r]) * F[r];
-        else y = ((cc0 * s0v[r] + cc1 * cur[lg]) + cc2 * prev[lg]) + ((cf * dtv[r]) * F[r]);
-        // store_with_ghosts into the strip
-        const float sz = a.sz;
-        const bool lo_i = ic <= 3, hi_i = ic >= n - 3, lo_k = k <= 3, hi_k = k >= m - 3;
-        put(out, ic, k, y);
-        if (lo_i) put(out, -ic, k, -y);
-        if (hi_i) put(out, 2 * n - ic, k, -y);
-        if (lo_k) {
-          put(out, ic, -k, sz * y);
-          if (lo_i) put(out, -ic, -k, -(sz * y));
-          if (hi_i) put(out, 2 * n - ic, -k, -(sz * y));
+        for (int r = 0; r < RB; r++) s0v[r] = F[r];   // the residual
+      } else {
+        R* const out = buf + (ne - at0) + own;
+#pragma unroll
+        for (int r = 0; r < RB; r++) {
+          R y;
+          if (a.j0 + t == 1) y = s0v[r] + (cf * dtv[r]) * F[r];
+          else y = ((cc0 * s0v[r] + cc1 * s1[r]) + cc2 * pv[r]) + ((cf * dtv[r]) * F[r]);
+          pv[r] = s1[r];
+          yv[r] = y;
+          if (t < nev - 1 && k0 + r <= m - 1) out[r * W] = y;
         }
-        if (hi_k) {
-          put(out, ic, 2 * m - k, sz * y);
-          if (lo_i) put(out, -ic, 2 * m - k, -(sz * y));
-          if (hi_i) put(out, 2 * n - ic, 2 * m - k, -(sz * y));
+        if (t < nev - 1) {
+#pragma unroll
+          for (int r = 0; r < RB; r++) {
+            if (k0 + r > m - 1) continue;
+            const R y = yv[r], z = a.sz * y;
+            const int at = r * W;
+            if (tiny) {
+              int i = ic, k = k0 + r;
+              asm volatile("" : "+v"(i), "+v"(k));   // not kept in registers between stages
+              const int ol = at - 2 * i, orr = at + 2 * (n - i), ob = -2 * k * W, ot = 2 * (m - k) * W;
+              const bool gl = i <= 3 && -i >= ilo, gr = i >= n - 3 && 2 * n - i < ilo + W;
+              if (gl) out[ol] = -y;
+              if (gr) out[orr] = -y;
+              if (k <= 3 && -k >= klo) {
+                out[at + ob] = z;
+                if (gl) out[ol + ob] = -z;
+                if (gr) out[orr + ob] = -z;
+              }
+              if (k >= m - 3 && 2 * m - k < klo + rows) {
+                out[at + ot] = z;
+                if (gl) out[ol + ot] = -z;
+                if (gr) out[orr + ot] = -z;
+              }
+              continue;
+            }
+            if (gx) out[at + gx] = -y;
+            if (gz[r]) {
+              out[at + gz[r]] = z;
+              if (gx) out[at + gz[r] + gx] = -z;
+            }
+          }
         }
       }
     }
-    __syncthreads();
-    pi = ci;
-    ci = oi;
+    if (t + 1 < nev) __syncthreads();
+    at0 = ne - at0;
   }
-  // core columns of the last two stages to global memory, with ghost images
-  const int cwc = c1 - c0, npts = cwc * (m - 1);
-  for (int e = tid; e < npts; e += nthr) {
-    const int k = 1 + e / cwc, i = c0 + (e - (k - 1) * cwc);
-    const int lg = (k + 3) * W + (i - lo);
-    store_with_ghosts<float>(s.Ocur, i, k, n, m, p, buf[ci * bsz + lg], a.sz);
-    if (s.Oprev) store_with_ghosts<float>(s.Oprev, i, k, n, m, p, buf[pi * bsz + lg], a.sz);
+  if (!col || ic < cx0 || ic >= cx1) return;
+#pragma unroll
+  for (int r = 0; r < RB; r++) {
+    const int k = k0 + r;
+    if (k < cz0 || k >= cz1) continue;
+    store_with_ghosts<R>(a.Ocur, ic, k, n, m, p, yv[r], a.sz);
+    if (a.Oprev) store_with_ghosts<R>(a.Oprev, ic, k, n, m, p, pv[r], a.sz);
+    if (a.res) a.res[IDX(ic, k, p)] = s0v[r];
   }
 }
 
@@ -1382,7 +1219,6 @@ static StageArgs<R> stage_base(Context& c, int l, bool fp32) {
       a.Drs[b][q] = (R)c.st.Drs[b][q]; a.Drss[b][q] = (R)c.st.Drss[b][q];
       a.Drrs[b][q] = (R)c.st.Drrs[b][q]; a.Drrss[b][q] = (R)c.st.Drrss[b][q];
     }
-  a.ivis0 = c.P.ivis == 0;
   if (!fp32) {
     a.vis = (const R*)L.v.vis; a.vxm = (const R*)L.v.vxxmzz; a.vxz = (const R*)L.v.vxz;
     a.vx = (const R*)L.v.vx; a.vz = (const R*)L.v.vz; a.rhs = (const R*)L.rhs; a.dts = (const R*)L.dts;
@@ -1393,147 +1229,240 @@ static StageArgs<R> stage_base(Context& c, int l, bool fp32) {
   return a;
 }
 
-template <typename R, bool IV0>
-static void launch_stage(Context& c, dim3 grd, dim3 blk, const StageArgs<R>& a) {
-  hipLaunchKernelGGL((k_stage<R, IV0>), grd, blk, 0, c.stream, a);
-}
-template <typename R>
-static void launch_stage(Context& c, dim3 grd, dim3 blk, const StageArgs<R>& a) {
-  if (c.P.ivis == 0) launch_stage<R, true>(c, grd, blk, a);
-  else launch_stage<R, false>(c, grd, blk, a);
-}
 template <typename R>
 static void launch_residual(Context& c, dim3 grd, dim3 blk, const StageArgs<R>& a, R* res, double* partial) {
   if (c.P.ivis == 0) hipLaunchKernelGGL((k_residual<R, true>), grd, blk, 0, c.stream, a, res, partial);
   else hipLaunchKernelGGL((k_residual<R, false>), grd, blk, 0, c.stream, a, res, partial);
 }
 
-// points per thread of the single-workgroup smoother, 0 when the level is
-// too large for it: beyond 4 points (isoviscous) the per-thread state no
-// longer fits in 128 VGPRs; with the full variable-viscosity operator one
-// workgroup is slower than a launch per stage beyond 2 points (FP32 level
-// 127x31: 248 us per 35-stage sweep against 35 x 4.9 us)
-static int small_ppt(int n, int m, bool iv0) {
-  const int npts = (n - 1) * (m - 1);
-  const int pmax = iv0 ? 4 : 2;
-  for (int ppt = 1; ppt <= pmax; ppt *= 2)
-    if (npts <= ppt * SMALL_THREADS) return ppt;
-  return 0;
+// ---------------------------------------------------------------------------
+// sweeps: tiling, launches
+// ---------------------------------------------------------------------------
+template <typename R, int EV, int RB>
+constexpr int sweep_threads() {
+  return sizeof(R) == 8 && EV == 0 && RB == 4 ? 512 : 1024;
 }
+static int sweep_threads_of(bool f32, int ev, int rb) { return !f32 && ev == 0 && rb == 4 ? 512 : 1024; }
 
-template <typename R, bool IV0, int PPT>
-static int launch_small_t(Context& c, size_t lds, const StageArgs<R>& a, R* err, R* res, int s, double cc,
-                          const RkcCoef& co) {
-  // set once per process (a thread-safe static initialisation)
-  static const hipError_t attr_rc = hipFuncSetAttribute((const void*)k_smooth_small<R, IV0, PPT>,
-                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)SMALL_LDS_BYTES);
-  PT_HIP(attr_rc);
-  hipLaunchKernelGGL((k_smooth_small<R, IV0, PPT>), dim3(1), dim3(SMALL_THREADS), lds, c.stream, a, err, res, s, cc,
-                     co);
-  return PT_OK;
-}
-template <typename R, bool IV0>
-static int launch_small_v(Context& c, int ppt, size_t lds, const StageArgs<R>& a, R* err, R* res, int s, double cc,
-                          const RkcCoef& co) {
-  switch (ppt) {
-    case 1: return launch_small_t<R, IV0, 1>(c, lds, a, err, res, s, cc, co);
-    case 2: return launch_small_t<R, IV0, 2>(c, lds, a, err, res, s, cc, co);
-    default: return launch_small_t<R, IV0, 4>(c, lds, a, err, res, s, cc, co);
-  }
-}
-
-// rows per thread of the column-blocked FP32 sweep: 4 when that keeps at
-// least half the workgroup busy with one column block per thread, 1 when
-// every interior point has a thread of its own, else 0
-static int cb_rows(int n, int m) {
-  const int b4 = (n - 1) * ((m - 1 + 3) / 4);
-  if (b4 <= SMALL_THREADS && 2 * b4 >= SMALL_THREADS) return 4;
-  return (n - 1) * (m - 1) <= SMALL_THREADS ? 1 : 0;
-}
-template <int RB>
-static int launch_cb_t(Context& c, size_t lds, const StageArgs<float>& a, float* err, float* res, int s, double cc,
-                       const RkcCoef& co) {
-  // set once per process (a thread-safe static initialisation)
-  static const hipError_t attr_rc = hipFuncSetAttribute((const void*)k_smooth_cb<RB>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                               (int)SMALL_LDS_BYTES);
-  PT_HIP(attr_rc);
-  hipLaunchKernelGGL(k_smooth_cb<RB>, dim3(1), dim3(SMALL_THREADS), lds, c.stream, a, err, res, s, rkc_f32(co, cc));
-  return PT_OK;
-}
-static int launch_cb(Context& c, int rb, size_t lds, const StageArgs<float>& a, float* err, float* res, int s,
-                     double cc, const RkcCoef& co) {
-  if (rb == 1) return launch_cb_t<1>(c, lds, a, err, res, s, cc, co);
-  return launch_cb_t<4>(c, lds, a, err, res, s, cc, co);
-}
-
-// strip sweep of an FP32 isoviscous level: core columns per workgroup and
-// stages per segment (cw == 0: not eligible).  The widest stage region (core
-// + 6 columns per further stage) spans at most the 64 column lanes; the
-// three strip buffers must fit LDS; rows are covered by 16 blocks of 4.
-// The most fused stages come first (9 stages on a 16-column core: 4
-// launches per 35-stage sweep): a workgroup's stage takes about the same
-// time for any core width, since its 16 waves wait on LDS and the barrier
-// rather than on issue, and each launch pays a strip load and store.
-struct StripCfg {
-  int cw = 0, ns = 0, W = 0;
+// the launch shape of `nev` evaluations on cw x ch cores
+struct SweepShape {
+  int w1, nrb, tcol, threads, nbx, nblk;
+  size_t lds;
 };
-static StripCfg strip_cfg(const LevelGeom& g) {
-  StripCfg sc;
-  if (g.m - 1 > STRIP_TY * STRIP_RB) return sc;
-  const size_t rows = (size_t)g.m + 7;
-  for (int ns = (STRIP_TX + 6 - 16) / 6; ns >= 2; ns--) {
-    for (int cw = STRIP_TX + 6 - 6 * ns; cw >= 16; cw -= 4) {
-      const int W = std::min(cw + 6 * ns, g.n + 7);
-      if (3 * (size_t)W * rows * sizeof(float) <= SMALL_LDS_BYTES) {
-        sc.cw = cw; sc.ns = ns; sc.W = W;
-        return sc;
-      }
-    }
-  }
-  return sc;
+static SweepShape sweep_shape(int n, int m, int cw, int ch, int rb, int nev, size_t elem) {
+  SweepShape s;
+  s.w1 = std::min(cw + 6 * (nev - 1), n - 1);
+  const int h1 = std::min(ch + 6 * (nev - 1), m - 1);
+  s.nrb = (h1 + rb - 1) / rb;
+  s.tcol = s.w1;
+  s.threads = (s.tcol * s.nrb + 63) & ~63;
+  s.nbx = (n - 1 + cw - 1) / cw;
+  s.nblk = s.nbx * ((m - 1 + ch - 1) / ch);
+  s.lds = 2 * elem * (size_t)(s.w1 + 8) * (s.nrb * rb + 8);
+  return s;
 }
 
-// one FP32 RKC1 sweep of level l as segments of fused stages.  The error
-// buffer holds S0 throughout; segments read one buffer pair and write the
-// other; the sweep result replaces the error buffer by a pointer swap.
-static int strip_sweep(Context& c, int l, const StripCfg& sc, double cpar, const RkcCoef& co) {
+// the operator's form on a level: general, isoviscous, or (FP32 levels >= 2
+// that one workgroup or column strips of at most 64 rows cover) isoviscous
+// with the factorised psi_xxzz
+static int sweep_form(const Context& c, int l, bool f32) {
+  if (c.P.ivis != 0) return 0;
+  if (!f32 || l < 2) return 1;
+  const LevelGeom& g = c.L[l].g;
+  const int npts = (g.n - 1) * (g.m - 1);
+  if (npts > 4096) return g.m - 1 <= 64 ? 2 : 1;
+  if (3 * sizeof(float) * c.L[l].nelem > SMALL_LDS_BYTES) return 1;
+  const int b4 = (g.n - 1) * ((g.m + 2) / 4);
+  return (b4 <= SMALL_THREADS && 2 * b4 >= SMALL_THREADS) || npts <= SMALL_THREADS ? 2 : 1;
+}
+
+// Modelled time (us) of one launch of `nev` evaluations; the model's terms
+// and the constants per operator form are a fit to 14,000 measured sweeps of
+// 30 levels from 7x7 to 1023x255 points (its choice is within 2% of the
+// measured best on 28 of them, within 9% on all):
+//   2.9            launch to launch
+//   fill, row      window loads per thread and per window row
+//   stage          an evaluation's latency (LDS round trip, barrier)
+//   wave           VALU time of a SIMD's wavefronts, per point of a thread
+//   lds            LDS time of a CU's wavefronts (29, 36, 50 reads for 1, 2, 4 points)
+struct SweepCost {
+  double fill, row, stage, wave, lds;
+};
+static double sweep_launch_us(const SweepCost& k, int n, int m, int cw, int ch, int rb, int nev,
+                              const SweepShape& s) {
+  constexpr int CUS = 256;
+  const int per = (s.nblk + CUS - 1) / CUS, rows = s.nrb * rb + 8;   // tiles per CU
+  double us = 2.9 + per * (k.fill * (s.w1 + 8) * rows / s.threads * ((s.threads + 255) / 256) + k.row * rows);
+  for (int h = 0; h < nev; h++) {
+    const int hh = std::min(ch + 6 * h, m - 1), ww = std::min(cw + 6 * h, n - 1);
+    const int nb = std::min(s.nrb, (hh + rb - 1) / rb + (h < nev - 1 && rb > 1 ? 1 : 0));
+    const int lanes = (ww < s.w1 && s.w1 >= 96 ? ww + 64 : s.w1) * nb;   // active row blocks, in whole wavefronts
+    const int waves = std::max(1, (lanes + 63) / 64) * per;
+    us += k.stage + k.wave * ((waves + 3) / 4) * rb + k.lds * waves * (rb == 1 ? 29 : rb == 2 ? 36 : 50) / 64;
+  }
+  return us;
+}
+
+// The tiling of a level's sweeps of s stages: the one with the least modelled
+// time.  Small tiles use more CUs and large ones recompute less overlap; more
+// stages per launch save launches and widen the overlap.  1024x256, 35
+// stages: 32x32 cores, 3 stages per launch, 2 points per thread (FP32 general
+// operator 150 us a sweep against 35 launches of one stage at 8.5 us; FP64
+// isoviscous 144 us against 35 x 6.0); 256x64: 16x4, 3, 1 (FP32 general, 15
+// stages: 30 us against 15 x 5.5); 32x32 FP64: one workgroup, all stages, 2
+// points per thread (49 us; one point per thread and a row of LDS reads per
+// point: 58).
+static SweepPlan sweep_plan(const Context& c, int l, bool f32, int s) {
+  const LevelGeom& g = c.L[l].g;
+  const int n = g.n, m = g.m, ev = sweep_form(c, l, f32);
+  const SweepCost cost = f32 ? (ev == 0   ? SweepCost{0.10, 0.01, 0.75, 0.21, 0.038}
+                                : ev == 1 ? SweepCost{0.18, 0.02, 0.31, 0.081, 0.008}
+                                          : SweepCost{0.15, 0.01, 0.46, 0.057, 0.006})
+                             : (ev == 0 ? SweepCost{0.034, 0.03, 0.60, 0.453, 0.015}
+                                        : SweepCost{0.21, 0.03, 0.59, 0.345, 0.013});
+  const size_t elem = f32 ? 4 : 8;
+  const int cws[] = {8, 12, 16, 24, 32, 48, 64, 96, 128, 192, 256, n - 1};
+  const int chs[] = {4, 8, 12, 16, 24, 32, 48, 64, m - 1};
+  // levels >= 2 may form the residual in the last launch
+  const int extra = l >= 2 ? 1 : 0;
+  SweepPlan best = {std::min(8, n - 1), std::min(4, m - 1), 1, 1};
+  double best_us = INFINITY;
+  for (int rb = 1; rb <= 4; rb *= 2)
+    for (int cw : cws)
+      for (int ch : chs) {
+        if (cw > n - 1 || ch > m - 1) continue;
+        for (int ns = 1; ns <= s; ns++) {
+          const int nseg = (s + ns - 1) / ns, base = s / nseg, rem = s % nseg;
+          if (base + (rem ? 1 : 0) != ns) continue;   // a larger ns with as many launches
+          const SweepShape widest = sweep_shape(n, m, cw, ch, rb, ns + extra, elem);
+          if (widest.threads > sweep_threads_of(f32, ev, rb) || widest.lds > SWEEP_LDS_BYTES) break;
+          double us = rem * sweep_launch_us(cost, n, m, cw, ch, rb, ns, sweep_shape(n, m, cw, ch, rb, ns, elem));
+          if (nseg > rem + 1)
+            us += (nseg - rem - 1) *
+                  sweep_launch_us(cost, n, m, cw, ch, rb, base, sweep_shape(n, m, cw, ch, rb, base, elem));
+          const int last = base + (f32 ? 0 : extra);
+          us += sweep_launch_us(cost, n, m, cw, ch, rb, last, sweep_shape(n, m, cw, ch, rb, last, elem));
+          if (us < best_us) {
+            best_us = us;
+            best = {cw, ch, ns, rb};
+          }
+        }
+      }
+  return best;
+}
+
+template <typename R>
+static SweepArgs<R> sweep_args(Context& c, int l, bool f32, const LevelRkc& rk, double cpar) {
+  SweepArgs<R> a;
+  std::memset(&a, 0, sizeof a);
+  const StageArgs<R> b = stage_base<R>(c, l, f32);
+  a.vis = b.vis; a.vxm = b.vxm; a.vxz = b.vxz; a.vx = b.vx; a.vz = b.vz; a.rhs = b.rhs; a.dts = b.dts;
+  a.n = b.n; a.m = b.m; a.pitch = b.pitch; a.sz = b.sz;
+  a.dr2 = b.dr2; a.dr3 = b.dr3; a.dr4 = b.dr4; a.ds2 = b.ds2; a.ds3 = b.ds3; a.ds4 = b.ds4;
+  a.drds = b.drds; a.dr2ds = b.dr2ds; a.drds2 = b.drds2; a.dr2ds2 = b.dr2ds2;
+  a.rdr2 = b.rdr2; a.rdr3 = b.rdr3; a.rdr4 = b.rdr4; a.rds2 = b.rds2; a.rds3 = b.rds3; a.rds4 = b.rds4;
+  a.rdrds = b.rdrds; a.rdr2ds = b.rdr2ds; a.rdrds2 = b.rdrds2; a.rdr2ds2 = b.rdr2ds2;
+  for (int q = 0; q < 3; q++) { a.w.d2[q] = b.D2[2 + q]; a.w.d3[q] = b.D3[2 - q]; }
+  for (int q = 0; q < 4; q++) a.w.d4[q] = b.D4[3 + q];
+  a.w.rs[0] = b.Drs[3][3]; a.w.rs[1] = b.Drs[3][4]; a.w.rs[2] = b.Drs[4][4];
+  for (int u = 0; u < 2; u++)
+    for (int q = 0; q < 3; q++) {
+      a.w.rrs[u * 3 + q] = b.Drrs[1 - u][2 + q];
+      a.w.rss[u * 3 + q] = b.Drss[2 + q][1 - u];
+    }
+  for (int q = 0; q < 3; q++) a.w.rrss[q] = b.Drrss[2][2 + q];
+  a.w.rrss[3] = b.Drrss[3][3]; a.w.rrss[4] = b.Drrss[3][4]; a.w.rrss[5] = b.Drrss[4][4];
+  for (int j = 0; j < SWEEP_MAX_STAGES; j++) {
+    a.c0[j] = (R)rk.cc[j]; a.c1[j] = (R)rk.mew[j]; a.c2[j] = (R)rk.vv[j]; a.cf[j] = (R)(rk.mewt[j] * cpar);
+  }
+  return a;
+}
+
+template <typename R, int EV, int RB, bool PW2>
+static int launch_sweep_t(Context& c, const SweepShape& s, const SweepArgs<R>& a) {
+  constexpr int NT = sweep_threads<R, EV, RB>();
   // set once per process (a thread-safe static initialisation)
-  static const hipError_t attr_rc = hipFuncSetAttribute((const void*)k_strip_cb, hipFuncAttributeMaxDynamicSharedMemorySize,
-                               (int)SMALL_LDS_BYTES);
+  static const hipError_t attr_rc = hipFuncSetAttribute((const void*)k_sweep<R, EV, RB, NT, PW2>,
+                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)SWEEP_LDS_BYTES);
   PT_HIP(attr_rc);
+  hipLaunchKernelGGL((k_sweep<R, EV, RB, NT, PW2>), dim3(s.nblk), dim3(s.threads), s.lds, c.stream, a);
+  return PT_OK;
+}
+template <typename R, int EV, bool PW2>
+static int launch_sweep_rb(Context& c, int rb, const SweepShape& s, const SweepArgs<R>& a) {
+  switch (rb) {
+    case 1: return launch_sweep_t<R, EV, 1, PW2>(c, s, a);
+    case 2: return launch_sweep_t<R, EV, 2, PW2>(c, s, a);
+    default: return launch_sweep_t<R, EV, 4, PW2>(c, s, a);
+  }
+}
+static int launch_sweep(Context& c, int l, int ev, int rb, const SweepShape& s, const SweepArgs<float>& a) {
+  (void)l;
+  if (ev == 0) return launch_sweep_rb<float, 0, true>(c, rb, s, a);
+  return ev == 1 ? launch_sweep_rb<float, 1, true>(c, rb, s, a) : launch_sweep_rb<float, 2, true>(c, rb, s, a);
+}
+static bool pow2(double x) {
+  int e;
+  return std::frexp(x, &e) == 0.5;
+}
+static int launch_sweep(Context& c, int l, int ev, int rb, const SweepShape& s, const SweepArgs<double>& a) {
+  const LevelGeom& g = c.L[l].g;
+  // all of the level's grid powers are products of dr and ds
+  const bool pw2 = pow2(g.dr) && pow2(g.ds) && pow2(g.dr4) && pow2(g.ds4) && pow2(g.dr2ds2);
+  if (ev == 0) return pw2 ? launch_sweep_rb<double, 0, true>(c, rb, s, a) : launch_sweep_rb<double, 0, false>(c, rb, s, a);
+  return pw2 ? launch_sweep_rb<double, 1, true>(c, rb, s, a) : launch_sweep_rb<double, 1, false>(c, rb, s, a);
+}
+
+// one RKC1 sweep of level l (PS/iterative_solver.f90:1418-1614), the residual
+// of its result into `res` when wanted.  The error buffer holds S0 throughout;
+// launches read one pair of work buffers and write the other, and the last
+// one's output replaces the error buffer by a pointer swap.  One tile that
+// covers the level reads and writes the error buffer alone.
+template <typename R>
+static int sweep_level(Context& c, int l, bool f32, const LevelRkc& rk, double cpar, R* res) {
   Level& L = c.L[l];
-  float** f[5] = {&L.ferr, &L.fB, &L.fC, &L.fD, &L.fE};
   const LevelGeom& g = L.g;
-  const int s = level_rkc(c, l, true).s;
-  const int nseg = (s + sc.ns - 1) / sc.ns, base = s / nseg, rem = s % nseg;
-  if (base < 2) {
-    set_error("strip sweep needs at least 2 stages per segment");
-    return PT_ERR_UNSUPPORTED;
+  R** f[5];
+  if constexpr (sizeof(R) == 4) {
+    R** q[5] = {&L.ferr, &L.fB, &L.fC, &L.fD, &L.fE};
+    std::copy(q, q + 5, f);
+  } else {
+    R** q[5] = {&L.err, &L.bufB, &L.bufC, &L.bufD, &L.bufE};
+    std::copy(q, q + 5, f);
   }
-  const int nblk = (g.n - 1 + sc.cw - 1) / sc.cw;
-  const size_t lds = 3 * (size_t)sc.W * (g.m + 7) * sizeof(float);
-  StageArgs<float> a = stage_base<float>(c, l, true);
-  StripArgs sa;
-  sa.S0 = *f[0]; sa.cw = sc.cw; sa.W = sc.W; sa.co = rkc_f32(co, cpar);
-  int rd = 1, wr = 3;   // read pair f[rd], f[rd+1]; write pair f[wr], f[wr+1]
-  int j0 = 1;
+  const SweepPlan& p = L.plan[f32];
+  const int ev = sweep_form(c, l, f32), s = rk.s;
+  const int nseg = (s + p.ns - 1) / p.ns, base = s / nseg, rem = s % nseg;
+  const int tk = l == 1 ? PT_K_RKC_STAGE_L1 : PT_K_RKC_STAGE_COARSE;
+  SweepArgs<R> a = sweep_args<R>(c, l, f32, rk, cpar);
+  a.cw = p.cw; a.ch = p.ch; a.S0 = *f[0];
+  int rd = 1, wr = 3, j0 = 1;
   for (int seg = 0; seg < nseg; seg++) {
-    const int len = base + (seg < rem ? 1 : 0), j1 = j0 + len - 1;
-    sa.j0 = j0; sa.j1 = j1;
-    sa.Gcur = *f[rd]; sa.Gprev = *f[rd + 1];
-    sa.Ocur = *f[wr]; sa.Oprev = (j1 == s) ? nullptr : *f[wr + 1];
-    hipLaunchKernelGGL(k_strip_cb, dim3(nblk), dim3(STRIP_TX, STRIP_TY), lds, c.stream, a, sa);
+    const int len = base + (seg < rem ? 1 : 0);
+    const bool end = seg == nseg - 1;
+    a.j0 = j0; a.ns = len; a.res = end ? res : nullptr;
+    const SweepShape sh = sweep_shape(g.n, g.m, p.cw, p.ch, p.rb, len + (a.res ? 1 : 0), sizeof(R));
+    if (sh.threads > sweep_threads_of(f32, ev, p.rb) || sh.lds > SWEEP_LDS_BYTES) {
+      set_error("sweep tile too large");
+      return PT_ERR_INVALID;
+    }
+    const bool alone = sh.nblk == 1 && nseg == 1;
+    a.Gcur = j0 == 1 ? *f[0] : *f[rd];
+    a.Gprev = j0 == 1 ? *f[0] : *f[rd + 1];
+    a.Ocur = alone ? *f[0] : *f[wr];
+    a.Oprev = end ? nullptr : *f[wr + 1];
+    a.nbx = sh.nbx; a.w1 = sh.w1; a.nrb = sh.nrb; a.tcol = sh.tcol;
+    if (c.timing) timer_begin(c, tk, (int64_t)len * (g.n - 1) * (g.m - 1));
+    PT_TRY(launch_sweep(c, l, ev, p.rb, sh, a));
+    if (c.timing) timer_end(c, tk);
+    if (alone) return PT_OK;
     std::swap(rd, wr);
-    j0 = j1 + 1;
+    j0 += len;
   }
-  std::swap(*f[0], *f[rd]);   // the last segment's output becomes the error buffer
+  std::swap(*f[0], *f[rd]);
   return PT_OK;
 }
 
-// first level of the fused sub-cycle, 0 when it does not apply: levels
-// ls..grids-1 are single-workgroup sweeps whose argument table fits the
-// kernel arguments, the coarse operator fits one workgroup, and in the mixed
-// path level ls-1 is an FP32 level (ls >= 3)
 static int launch_coarse_apply_wg(Context& c, const float* rhs, float* err, int n, int m, int pitch, float sz) {
   // set once per process (a thread-safe static initialisation)
   static const hipError_t attr_rc = hipFuncSetAttribute((const void*)k_coarse_apply_wg, hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -1548,16 +1477,13 @@ static int launch_coarse_apply_wg(Context& c, const float* rhs, float* err, int 
   return PT_OK;
 }
 
-// iterate_stream (RKC1, Nmulti sweeps) followed by compute_residual
-// (PS/iterative_solver.f90:1418-1614, 415-448).  `s0zero` runs the smoother
-// on a correction that starts from zero (mixed precision).
-// residual of the smoothed field
+// residual of the smoothed field (compute_residual, PS/iterative_solver.f90:415-448)
 template <typename R>
 static int smoothed_residual(Context& c, int l, dim3 grd, dim3 blk, bool fp32, bool l1_sum) {
   Level& L = c.L[l];
   StageArgs<R> a = stage_base<R>(c, l, fp32);
   a.Sx = fp32 ? (R*)L.ferr : (R*)L.err;
-  R* res = fp32 ? (R*)L.fB : (R*)L.res;   // FP32 residual reuses the B buffer
+  R* res = fp32 ? (R*)L.fres : (R*)L.res;
   int nb = grd.x * grd.y;
   launch_residual<R>(c, grd, blk, a, res, c.red);
   if (l1_sum) {
@@ -1568,117 +1494,48 @@ static int smoothed_residual(Context& c, int l, dim3 grd, dim3 blk, bool fp32, b
   return PT_OK;
 }
 
+// iterate_stream (Nmulti sweeps) and the residual after it where it is read
+// (PS/iterative_solver.f90:1418-1614, 415-448)
 template <typename R>
 static int iterate_stream_t(Context& c, int l, int p, bool fp32, bool l1_sum) {
   Level& L = c.L[l];
   const LevelGeom& g = L.g;
-  const LevelRkc rk = level_rkc(c, l, fp32);
-  const int s = rk.s;
   dim3 blk(TX, TZ), grd((g.n - 1 + TX - 1) / TX, (g.m - 1 + TZ * PZ - 1) / (TZ * PZ));
-  R* err = fp32 ? (R*)L.ferr : (R*)L.err;
-  R* B = fp32 ? (R*)L.fB : (R*)L.bufB;
-  R* Cb = fp32 ? (R*)L.fC : (R*)L.bufC;
-  const bool timed = c.timing;
-  const int tk = l == 1 ? PT_K_RKC_STAGE_L1 : PT_K_RKC_STAGE_COARSE;
-  const size_t lds = 3 * L.nelem * sizeof(R);
-  const int ppt = small_ppt(g.n, g.m, c.P.ivis == 0);
+  // the residual is read by the stop test (level 1) and by the restriction
+  // when the cycle goes down from here
+  const bool want_res = l1_sum || c.cyc[p + 1] > c.cyc[p];
   if constexpr (sizeof(R) == 8) {
     if (c.P.RKC1 == 0) {
       // RK1: per iteration F = stream_space(S0) into B, then the update
+      const int tk = l == 1 ? PT_K_RKC_STAGE_L1 : PT_K_RKC_STAGE_COARSE;
       const int dir = c.cyc[p + 1] > c.cyc[p] ? 0 : 1;
       dim3 b16(64, 4), gi((g.n - 1 + 63) / 64, (g.m - 1 + 3) / 4);
       for (int it = 1; it <= c.P.Nmulti; it++) {
         const int ntemp = c.P.Nmulti - it + 1;
         const double temp = std::cos((double)(2 * ntemp - 1) * 3.1415926535897932 / (double)(2 * c.P.Nmulti));
         StageArgs<R> a = stage_base<R>(c, l, false);
-        a.Sx = err;
-        if (timed) timer_begin(c, tk, (int64_t)(g.n - 1) * (g.m - 1));
-        launch_residual<R>(c, grd, blk, a, B, c.red);
-        hipLaunchKernelGGL(k_rk1_update, gi, b16, 0, c.stream, (double*)err, (const double*)B, L.dts, L.ratio, g.n,
+        a.Sx = L.err;
+        if (c.timing) timer_begin(c, tk, (int64_t)(g.n - 1) * (g.m - 1));
+        launch_residual<R>(c, grd, blk, a, L.bufB, c.red);
+        hipLaunchKernelGGL(k_rk1_update, gi, b16, 0, c.stream, L.err, (const double*)L.bufB, L.dts, L.ratio, g.n,
                            g.m, g.pitch, temp, dir, (double)a.sz);
-        if (timed) timer_end(c, tk);
+        if (c.timing) timer_end(c, tk);
       }
       return smoothed_residual<R>(c, l, grd, blk, fp32, l1_sum);
     }
   }
-  if constexpr (sizeof(R) == 4) {
-    // FP32 isoviscous levels too large for one workgroup: strip sweeps
-    const StripCfg sc = strip_cfg(g);
-    if (l >= 2 && c.P.ivis == 0 && ppt == 0 && sc.cw > 0 && !l1_sum) {
-      const RkcCoef co = rkc_coef(rk);
-      for (int it = 1; it <= c.P.Nmulti; it++) {
-        int ntemp = c.P.Nmulti - it + 1;
-        double temp = (c.P.Nmulti > 1) ? (c.P.c_2 - c.P.c_1) * (double)(ntemp - 1) / (double)(1 - c.P.Nmulti) : 0.0;
-        PT_TRY(strip_sweep(c, l, sc, temp + c.P.c_2, co));
-      }
-      StageArgs<R> a = stage_base<R>(c, l, fp32);
-      a.Sx = (R*)L.ferr;
-      launch_residual<R>(c, grd, blk, a, (R*)L.fB, c.red);
-      (void)p;
-      return PT_OK;
-    }
-  }
-  if (l >= 2 && ppt > 0 && lds <= SMALL_LDS_BYTES && !l1_sum) {
-    // whole sweep + residual in one workgroup, buffers in LDS
-    const RkcCoef co = rkc_coef(rk);
-    R* res = fp32 ? (R*)L.fB : (R*)L.res;
-    for (int it = 1; it <= c.P.Nmulti; it++) {
-      int ntemp = c.P.Nmulti - it + 1;
-      double temp = (c.P.Nmulti > 1) ? (c.P.c_2 - c.P.c_1) * (double)(ntemp - 1) / (double)(1 - c.P.Nmulti) : 0.0;
-      double cc = temp + c.P.c_2;
-      StageArgs<R> a = stage_base<R>(c, l, fp32);
-      // the residual buffer aliases fB in FP32 mode: the fused kernel keeps its
-      // RKC buffers in LDS, so fB is free
-      if constexpr (sizeof(R) == 4) {
-        const int rb = cb_rows(g.n, g.m);
-        if (c.P.ivis == 0 && rb > 0) {
-          PT_TRY(launch_cb(c, rb, lds, a, err, res, s, cc, co));
-          continue;
-        }
-      }
-      if (c.P.ivis == 0) PT_TRY((launch_small_v<R, true>(c, ppt, lds, a, err, res, s, cc, co)));
-      else PT_TRY((launch_small_v<R, false>(c, ppt, lds, a, err, res, s, cc, co)));
-    }
-    (void)p;
-    return PT_OK;
-  }
+  const LevelRkc rk = level_rkc(c, l, fp32);
+  // the residual of levels >= 2 comes out of the sweep's last launch; level
+  // 1's carries the L1 sum, and the residual of strip-covered isoviscous
+  // FP32 levels is the unfactorised form's
+  const bool fuse = want_res && l >= 2 && !(sweep_form(c, l, fp32) == 2 && (g.n - 1) * (g.m - 1) > 4096);
+  R* res = fp32 ? (R*)L.fres : (R*)L.res;
   for (int it = 1; it <= c.P.Nmulti; it++) {
     int ntemp = c.P.Nmulti - it + 1;
     double temp = (c.P.Nmulti > 1) ? (c.P.c_2 - c.P.c_1) * (double)(ntemp - 1) / (double)(1 - c.P.Nmulti) : 0.0;
-    double cc = temp + c.P.c_2;
-    StageArgs<R> a = stage_base<R>(c, l, fp32);
-    // stage 1: S1 = S0 + mewt1*c*dt*F(S0) -> B
-    a.Sx = err; a.S0 = err; a.S2 = err; a.Y = B; a.stage1 = 1; a.cf = (R)(rk.mewt[1] * cc);
-    if (timed) timer_begin(c, tk, (int64_t)(g.n - 1) * (g.m - 1));
-    launch_stage<R>(c, grd, blk, a);
-    if (timed) timer_end(c, tk);
-    // rotating buffers: S1 in `cur`, S2 in `prev`; Y goes to the S2 buffer
-    // except at stage 2 (S2 aliases S0) and at the last stage (Y -> err)
-    R* cur = B;
-    R* prev = err;   // S2 = S0 interior at stage 2
-    R* spare = Cb;
-    for (int j = 2; j <= s; j++) {
-      a.stage1 = 0;
-      a.Sx = cur; a.S0 = err; a.S2 = prev;
-      a.c0 = (R)rk.cc[j]; a.c1 = (R)rk.mew[j]; a.c2 = (R)rk.vv[j]; a.cf = (R)(rk.mewt[j] * cc);
-      R* out;
-      if (j == s) out = err;
-      else if (prev == err) out = spare;
-      else out = prev;
-      a.Y = out;
-      if (timed) timer_begin(c, tk, (int64_t)(g.n - 1) * (g.m - 1));
-      launch_stage<R>(c, grd, blk, a);
-      if (timed) timer_end(c, tk);
-      if (j < s) {
-        R* np = cur;
-        cur = out;
-        prev = np;
-        spare = (out == spare) ? nullptr : spare;
-      }
-    }
+    PT_TRY(sweep_level<R>(c, l, fp32, rk, temp + c.P.c_2, fuse && it == c.P.Nmulti ? res : nullptr));
   }
-  (void)p;
-  return smoothed_residual<R>(c, l, grd, blk, fp32, l1_sum);
+  return want_res && !fuse ? smoothed_residual<R>(c, l, grd, blk, fp32, l1_sum) : PT_OK;
 }
 
 // smoother_vis (PS/smoother.f90:454-580) on the field set `vs` of level l
@@ -1879,7 +1736,7 @@ static int visit(Context& c, int p, bool mixed) {
       hipLaunchKernelGGL((k_restrict<double, float>), grid2(L.g.n - 1, L.g.m - 1, b16), b16, 0, c.stream, F.res,
                          F.g.pitch, L.frhs, L.g.n, L.g.m, L.g.pitch);
     else
-      hipLaunchKernelGGL((k_restrict<float, float>), grid2(L.g.n - 1, L.g.m - 1, b16), b16, 0, c.stream, F.fB,
+      hipLaunchKernelGGL((k_restrict<float, float>), grid2(L.g.n - 1, L.g.m - 1, b16), b16, 0, c.stream, F.fres,
                          F.g.pitch, L.frhs, L.g.n, L.g.m, L.g.pitch);
   }
   if (l < t.grids) {
@@ -1909,7 +1766,7 @@ static int visit(Context& c, int p, bool mixed) {
       StageArgs<float> a = stage_base<float>(c, l, true);
       a.Sx = L.ferr;
       dim3 blk(TX, TZ), grd((L.g.n - 1 + TX - 1) / TX, (L.g.m - 1 + TZ * PZ - 1) / (TZ * PZ));
-      launch_residual<float>(c, grd, blk, a, L.fB, c.red);
+      launch_residual<float>(c, grd, blk, a, L.fres, c.red);
     } else {
       PT_TRY(iterate_stream_t<float>(c, l, p, true, false));
     }
@@ -1970,15 +1827,16 @@ static int level1_residual(Context& c, double* resmag1) {
   return PT_OK;
 }
 
-// The level buffers whose roles rotate: a strip sweep swaps its level's
-// error buffer with a work buffer, so a cycle may start from one of a few
+// The level buffers whose roles rotate: a sweep of several tiles swaps its
+// level's error buffer with a work buffer, so a cycle may start from one of a few
 // arrangements, and a replay must leave the pointers as the eager launches
 // would have.
 static void buffer_roles(Context& c, std::vector<void*>& out) {
   out.clear();
   for (int l = 1; l <= c.T.grids; l++) {
     Level& L = c.L[l];
-    out.insert(out.end(), {(void*)L.ferr, (void*)L.fB, (void*)L.fC, (void*)L.fD, (void*)L.fE});
+    out.insert(out.end(), {(void*)L.ferr, (void*)L.fB, (void*)L.fC, (void*)L.fD, (void*)L.fE, (void*)L.err,
+                           (void*)L.bufB, (void*)L.bufC, (void*)L.bufD, (void*)L.bufE});
   }
 }
 static void restore_roles(Context& c, const std::vector<void*>& v) {
@@ -1986,7 +1844,9 @@ static void restore_roles(Context& c, const std::vector<void*>& v) {
   for (int l = 1; l <= c.T.grids; l++) {
     Level& L = c.L[l];
     float** f[5] = {&L.ferr, &L.fB, &L.fC, &L.fD, &L.fE};
+    double** d[5] = {&L.err, &L.bufB, &L.bufC, &L.bufD, &L.bufE};
     for (float** q : f) *q = (float*)v[j++];
+    for (double** q : d) *q = (double*)v[j++];
   }
 }
 
@@ -2154,7 +2014,7 @@ int solver_alloc(Context& c) {
     g.dr2ds2 = t.dr2ds2g[l];
     L.nelem = (size_t)(g.n + 7) * (g.m + 7);
     size_t b = sizeof(double) * L.nelem, f = sizeof(float) * L.nelem;
-    DALLOC(L.err, b); DALLOC(L.bufB, b); DALLOC(L.bufC, b); DALLOC(L.rhs, b); DALLOC(L.res, b);
+    DALLOC(L.err, b); DALLOC(L.bufB, b); DALLOC(L.bufC, b); DALLOC(L.bufD, b); DALLOC(L.bufE, b); DALLOC(L.rhs, b); DALLOC(L.res, b);
     DALLOC(L.dts, b); DALLOC(L.ratio, b); DALLOC(L.vis_static, b);
     VisSet* sets[2] = {&L.v, &L.vs};
     for (VisSet* s : sets) {
@@ -2162,10 +2022,12 @@ int solver_alloc(Context& c) {
       DALLOC(s->vxz, b); DALLOC(s->vxxpzz, b); DALLOC(s->vxxmzz, b); DALLOC(s->vsmooth, b);
     }
     if (c.P.precision == PT_PREC_MIXED) {
-      DALLOC(L.ferr, f); DALLOC(L.fB, f); DALLOC(L.fC, f); DALLOC(L.fD, f); DALLOC(L.fE, f); DALLOC(L.frhs, f);
+      DALLOC(L.ferr, f); DALLOC(L.fB, f); DALLOC(L.fC, f); DALLOC(L.fD, f); DALLOC(L.fE, f); DALLOC(L.fres, f); DALLOC(L.frhs, f);
       DALLOC(L.fdts, f); DALLOC(L.fvis, f); DALLOC(L.fvxm, f); DALLOC(L.fvxz, f); DALLOC(L.fvx, f); DALLOC(L.fvz, f);
     }
   }
+  const bool f32 = c.P.precision == PT_PREC_MIXED;
+  for (int l = 1; l < t.grids && c.P.iterate == 1; l++) c.L[l].plan[f32] = sweep_plan(c, l, f32, level_rkc(c, l, f32).s);
   if (c.P.precision == PT_PREC_MIXED) DALLOC(c.dres64, sizeof(double) * c.L[1].nelem);
   DALLOC(c.d_info, sizeof(int32_t));
   if (c.P.iterate == 1) {   // the coarsest-grid operator of the multigrid path
@@ -2197,7 +2059,7 @@ int solver_alloc(Context& c) {
 int solver_free(Context& c) {
   for (int l = 1; l <= c.T.grids; l++) {
     Level& L = c.L[l];
-    void* ps[] = {L.err, L.bufB, L.bufC, L.rhs, L.res, L.dts, L.ratio, L.vis_static, L.v.vis, L.v.vx, L.v.vz,
+    void* ps[] = {L.err, L.bufB, L.bufC, L.bufD, L.bufE, L.fres, L.rhs, L.res, L.dts, L.ratio, L.vis_static, L.v.vis, L.v.vx, L.v.vz,
                   L.v.vxx, L.v.vzz, L.v.vxz, L.v.vxxpzz, L.v.vxxmzz, L.v.vsmooth, L.vs.vis, L.vs.vx, L.vs.vz,
                   L.vs.vxx, L.vs.vzz, L.vs.vxz, L.vs.vxxpzz, L.vs.vxxmzz, L.vs.vsmooth, L.ferr, L.fB, L.fC, L.fD, L.fE,
                   L.frhs, L.fdts, L.fvis, L.fvxm, L.fvxz, L.fvx, L.fvz};
