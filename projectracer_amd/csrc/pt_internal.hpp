@@ -88,6 +88,11 @@ struct Level {
   SweepPlan plan[2];              // tiling of the level's RKC1 sweeps: FP64, FP32
 };
 
+// a filter loop's tiles: core size, passes per launch
+struct FilterPlan {
+  int cw, ch, K;
+};
+
 struct KTimer {
   hipEvent_t beg[1024], end[1024];
   int n = 0;
@@ -144,12 +149,14 @@ struct Context {
   double* cellsum;          // 27 per cell: (T*w, C*w, w) for the 3x3 neighbour nodes
   double *TxS, *CxS;        // halo-5 scratch fields for the filters
   int32_t* d_flags;         // [0]=tracer outside domain, [1]=tracer more than one cell from its slot's cell
-  // device-driven filter loops: control (done flag, pass count), its pinned
-  // host mirror, and the ring of per-check smoothness maxima (FP64 bit
-  // patterns); filter_on_device is false when PT_FILTER_HOST=1 at pt_create
+  // device-driven filter loops: control (deciding launch, pass count, buffer
+  // of the result), its pinned host mirror, the checks' partial maxima per
+  // tile (two launches') and, for many tiles, their maxima; the tilings of the
+  // T and C loops; filter_on_device is false when PT_FILTER_HOST=1 at pt_create
   int32_t* d_fctl = nullptr;
   int32_t* h_fctl = nullptr;
-  unsigned long long* d_fsm = nullptr;
+  double *d_fpart = nullptr, *d_fred = nullptr;
+  FilterPlan filter[2];
   bool filter_on_device = true;
   int hint_comp = 0, hint_temp = 0;   // pass counts of the previous C / T filter loops
   // reductions

@@ -27,6 +27,7 @@
 #include <type_traits>
 #include <vector>
 #include "pt_internal.hpp"
+#include "pt_quotient.hpp"
 
 namespace pt {
 
@@ -314,19 +315,6 @@ struct SweepArgs {
   R c0[SWEEP_MAX_STAGES], c1[SWEEP_MAX_STAGES], c2[SWEEP_MAX_STAGES], cf[SWEEP_MAX_STAGES];
 };
 
-// s / d, correctly rounded, from rd = RN(1/d).  PW2: d is a power of two and
-// the product is the quotient.  Otherwise two residual corrections: the first
-// leaves q within one unit of the quotient, and then the second rounds it
-// correctly (Markstein's theorem).  A quotient that overflows is returned as
-// it is (the correction of an infinity would be NaN).
-template <bool PW2>
-__device__ __forceinline__ double quot(double s, double d, double rd) {
-  const double q0 = s * rd;
-  if constexpr (PW2) return q0;
-  const double q1 = __fma_rn(__fma_rn(-q0, d, s), rd, q0);
-  const double q2 = __fma_rn(__fma_rn(-q1, d, s), rd, q1);
-  return fabs(q0) < INFINITY ? q2 : q0;
-}
 template <bool PW2>
 __device__ __forceinline__ float quot(float s, float d, float rd) { (void)d; return s * rd; }
 
@@ -1400,10 +1388,6 @@ static int launch_sweep(Context& c, int l, int ev, int rb, const SweepShape& s, 
   (void)l;
   if (ev == 0) return launch_sweep_rb<float, 0, true>(c, rb, s, a);
   return ev == 1 ? launch_sweep_rb<float, 1, true>(c, rb, s, a) : launch_sweep_rb<float, 2, true>(c, rb, s, a);
-}
-static bool pow2(double x) {
-  int e;
-  return std::frexp(x, &e) == 0.5;
 }
 static int launch_sweep(Context& c, int l, int ev, int rb, const SweepShape& s, const SweepArgs<double>& a) {
   const LevelGeom& g = c.L[l].g;

@@ -15,9 +15,9 @@
 //   k_reorder        keeps the tracer SoA in cell order (ID map for host copies)
 //   k_sym_* / k_t_*  enforceBCs / extendT / enforceBCs_comp
 //                    (PS/energy.f90:558-630, PS/composition.f90:1279-1292)
-//   k_smoothness / k_filter
-//                    smoother_time / smoother_time_T Richardson passes
-//                    (PS/smoother.f90:582-672, 75-139)
+//   k_filter_passes  smoother_time / smoother_time_T: checks and Richardson passes,
+//                    several per launch on LDS tiles (PS/smoother.f90:582-672,
+//                    75-139); k_smoothness / k_filter: the host-driven loop's
 //   k_conduct_*      load_conductivity_array (PS/energy.f90:59-86)
 //   k_source         tracer_space_uniform (PS/energy.f90:135-151)
 //   k_itab           compute_derivatives for u, w and the source into one
@@ -29,6 +29,7 @@
 #include <cstring>
 #include <algorithm>
 #include "pt_internal.hpp"
+#include "pt_quotient.hpp"
 
 namespace pt {
 
@@ -586,227 +587,579 @@ static void filter_pass(Context& c, const double* T0, double* out, int h, double
 // ---------------------------------------------------------------------------
 // Filter loops driven on the device.  The reference checks the field's
 // smoothness before every pass and stops at the first check below the
-// threshold (PS/smoother.f90:582-672).  Here one kernel per pass does both
-// halves of a loop iteration on its input field: the check (a partial
-// maximum per check workgroup, stored in the pass's slot of a ring) and the
-// pass itself, written to the other buffer.  The pass is speculative: every
-// workgroup of the next pass kernel reduces the partials (max is order-free
-// and exact) and, when the check is below the threshold, the kernel records
-// the pass count and raises the `done` flag instead of going on, so the
-// field the loop returns is the input of the pass whose check succeeded, as
-// in the reference.  No atomics: 256 same-address atomics per pass cost more
-// than the pass itself.  The host enqueues pass kernels in batches without
-// waiting; once `done` is set every later kernel returns at once.
-// Passes alternate between two buffers; each writes its field's ghost
-// images itself (the reference's enforceBCs / enforceBCs_comp after the pass).
+// threshold (PS/smoother.f90:582-672).  k_filter_passes makes K passes per
+// launch on tiles of the nodes in LDS (temporal blocking): pass t of a launch
+// is made on the tile's core widened by 2 nodes for every pass still to come,
+// so tiles exchange nothing within a launch, and the check before each pass
+// (a maximum, so its order is free) is taken on the tile's own nodes and left
+// as one partial maximum per tile and pass.  Every tile of the next launch
+// reduces those maxima.  When one of the K checks is below the threshold, the
+// launch repeats the previous launch's passes up to that check from the field
+// it started from, which is the field the reference stops with, and raises
+// the done flag; otherwise it makes the next K passes.  Three buffers rotate,
+// so the field a launch started from is intact in the next.  The host
+// enqueues launches in batches without waiting.
+//
+// Only the nodes 0..nx x 0..nz are read: ghost values are the mirror images of
+// node values (enforceBCs_comp; T: 2 T_wall + heating - image below and above),
+// formed where they are used, and written with the last pass's result.
+//
+// The reference checks C (halo 5) through a dummy with the halo-3 shape
+// (PS/smoother.f90:79, :602): sequence association makes it read the storage
+// with row length nx+7 instead of P = nx+11, so a check point and its
+// neighbours one row away lie 4 columns apart per row, and points in the
+// ghost columns are compared with the other end of their row.  A tile checks
+// its nodes (and the ghost rows below them); the ghost columns are checked by
+// one extra tile per band of rows, which keeps a strip along each side wall.
+//
+// One pass per launch (latency-bound: a launch to launch gap, a round trip
+// to memory for the field and one for the previous check) took 5.6 us and 1.5
+// us of gap at 1024x256.  Eight passes per launch, bound by the FP64 units and
+// LDS of the CUs (2.4 times the nodes for the overlap) and by 8 us per launch,
+// take 2.9 us each.
 // ---------------------------------------------------------------------------
-// At most this many workgroups of a pass kernel take a share of the check,
-// striding over its points, each leaving one partial maximum.
-constexpr int SC_BLOCKS = 256;
-constexpr int FSLOTS = 64;   // ring of check slots, SC_BLOCKS partial maxima (FP64 bit patterns) each
-
-__global__ void k_filter_init(int32_t* ctl, unsigned long long* sm) {
-  const int t = threadIdx.x;
-  if (t < 4) ctl[t] = 0;
-  for (int u = t; u < FSLOTS * SC_BLOCKS; u += blockDim.x) sm[u] = 0ull;
-}
+constexpr int FILTER_KMAX = 8;      // passes per launch
+constexpr int FILTER_RB = 5;        // nodes per thread, vertically adjacent
+constexpr int FILTER_THREADS = 1024;
+constexpr int FILTER_LDS_BYTES = 158 * 1024;   // dynamic: two windows and the checks
+constexpr int FILTER_MAX_PART = 1024;   // tiles whose partial maxima every tile reduces itself
 
 struct FilterArgs {
   int nx, nz, h, p;
-  double dr, ds, dr2, ds2;
-  double D1[5], D2[5];
-  int clamp01;          // C: clamp to [0,1], symmetric ghosts (enforceBCs_comp)
-  // T (clamp01 == 0): enforceBCs with the isothermal / insulating walls
+  double dr2, ds2, rdr2, rds2;
+  double d2[3];         // D2 at offsets 0, 1, 2
+  // T: enforceBCs with the isothermal / insulating walls
   int Tbot;
   double Tb, Tt, two_over_d20, H, Htype;
   const double* Cvis;   // halo 5, for the heating term of the T wall ghosts
-  int check_h, check_p; // the check's view of the field: halo and row pitch
+  double delta;
+  // tiles: core cw x ch, nbx x nbz of them, then (C) nbz edge tiles of two
+  // strips of `strip` columns
+  int cw, ch, nbx, nbz, strip, ntile;
+  int K;                // passes per launch
+  int pitch, rows;      // LDS window
+  int w1, nrb;          // columns and row blocks of the first pass's region
 };
 
+struct FilterLaunch {
+  const double *in, *prev;      // this launch's field; the one the previous launch started from
+  double* out;
+  int32_t* ctl;                 // deciding launch (0: none yet), passes made, buffer of the result
+  const double* part_prev;      // the previous launch's partial maxima, K per tile (one set when reduced)
+  double* part;
+  int nprev;                    // sets in part_prev; 0: first launch
+  int k, kprev;                 // passes of this launch and of the previous one, at most FilterArgs::K
+  int jprev;                    // passes made before the previous launch
+  int launch, out_id, prev_id;  // launch number from 1; buffer numbers
+  double cd[FILTER_KMAX], cdp[FILTER_KMAX];   // c dts of this launch's and of the previous launch's passes
+};
 
-// Pass j of the loop, in -> out, on a (64, 4) block grid over the nodes
-// 0..nx x 0..nz.  First the decision on the previous kernel's check (the
-// check before pass j-1, in slot prev): below the threshold, the loop ends
-// with j-2 passes made.  Otherwise: the check before pass j (the max
-// 5-neighbour jump of `in` viewed with halo check_h and pitch check_p,
-// smoothness in PS/smoother.f90:75-95, over i = 0..nx-1, k = 1..nz-1) into
-// slot cur, and the pass (one Richardson pass, smoother_space at every node,
-// then the ghost images) into out.
-__global__ void __launch_bounds__(256) k_filter_pass(const double* in, double* out, FilterArgs a, int32_t* ctl,
-                                                     unsigned long long* sm, int prev, int cur, int pass,
-                                                     double cdts, double delta) {
-  const int bid = blockIdx.y * gridDim.x + blockIdx.x;
-  const int tid = threadIdx.y * blockDim.x + threadIdx.x;
-  const int nx = a.nx, nz = a.nz, h = a.h, p = a.p;
-  // XCD-aware tiles: workgroups are dispatched round-robin over the 8 XCDs
-  // (bid % 8); each XCD gets a contiguous band of tiles, the same every
-  // pass, so a tile's field and most of its halo stay in that XCD's L2
-  const int nblk = (int)(gridDim.x * gridDim.y);
-  const int q8 = nblk / 8, r8 = nblk % 8, xcd = bid % 8;
-  const int lb = xcd * q8 + min(xcd, r8) + bid / 8;
-  const int tx = lb % (int)gridDim.x, ty = lb / (int)gridDim.x;
-  const int i = tx * blockDim.x + threadIdx.x, k = ty * blockDim.y + threadIdx.y;
-  const bool node = i <= nx && k <= nz;
-  const int ncheck = min(nblk, SC_BLOCKS);
-  // The control word, the previous check and every load of `in` this
-  // thread needs are issued together, before the decision: the loads do
-  // not depend on it, and a kernel after the loop's end only reads.
-  const int32_t done = ctl[0];
-  // the previous check: one partial maximum per check workgroup
-  const double prev_part = pass > 1 && tid < ncheck ? __longlong_as_double((long long)sm[(long)prev * SC_BLOCKS + tid])
-                                                      : 0.0;
-  double y = 0.0;
-  if (node) {
-    auto F = [&](int u, int v) { return in[(long)(v + h) * p + (u + h)]; };
-    double sr = 0.0, ss = 0.0, srr = 0.0, sss = 0.0;
-    for (int q = -2; q <= 2; q++) sr = sr + a.D1[q + 2] * F(i + q, k);
-    for (int q = -2; q <= 2; q++) ss = ss + a.D1[q + 2] * F(i, k + q);
-    for (int q = -2; q <= 2; q++) srr = srr + a.D2[q + 2] * F(i + q, k);
-    for (int q = -2; q <= 2; q++) sss = sss + a.D2[q + 2] * F(i, k + q);
-    double Tr = sr / a.dr, Ts = ss / a.ds, Trr = srr / a.dr2, Tss = sss / a.ds2;
-    double Tx = Tr / 1.0, Tz = Ts / 1.0;
-    double Txx = (Trr - Tx * 0.0) / 1.0, Tzz = (Tss - Tz * 0.0) / 1.0;
-    double temp = Txx + Tzz;
-    y = F(i, k) + cdts * temp;
-  }
-  double d = 0.0;
-  if (bid < ncheck) {
-    const long npts = (long)nx * (nz - 1);
-    auto G = [&](int u, int v) { return in[(long)(v + a.check_h) * a.check_p + (u + a.check_h)]; };
-    // with a full set of check workgroups, the 32 on each XCD stride over
-    // that XCD's eighth of the points, near its band of tiles
-    long e0 = (long)bid * 256 + tid, e_end = npts, estride = (long)ncheck * 256;
-    if (ncheck == SC_BLOCKS) {
-      const int x = bid % 8, jx = bid / 8;
-      e0 = npts * x / 8 + (long)jx * 256 + tid;
-      e_end = npts * (x + 1) / 8;
-      estride = (long)(SC_BLOCKS / 8) * 256;
-    }
-    for (long e = e0; e < e_end; e += estride) {
-      const int kk = 1 + (int)(e / nx), ii = (int)(e - (long)(kk - 1) * nx);
-      const double t = G(ii, kk);
-      const double a1 = fabs(G(ii, kk - 1) - t), a2 = fabs(G(ii + 1, kk - 1) - t), a3 = fabs(G(ii + 1, kk) - t),
-                   a4 = fabs(G(ii, kk + 1) - t), a5 = fabs(G(ii + 1, kk + 1) - t);
-      d = fmax(d, fmax(fmax(fmax(fmax(a1, a2), a3), a4), a5));
-    }
-  }
-  if (done) return;
-  // both block maxima at once: the previous check's (the decision) and this
-  // pass's check (this block's partial)
-  __shared__ double red[2][4];
-  double pm = prev_part;
+__device__ __forceinline__ int mirror(int i, int n) { return n - abs(n - abs(i)); }   // -n <= i <= 2 n
+
+// maximum over a wavefront, in every lane
+__device__ __forceinline__ double wave_max_f64(double d) {
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    pm = fmax(pm, __shfl_xor(pm, o, 64));
-    d = fmax(d, __shfl_xor(d, o, 64));
+  for (int o = 32; o > 0; o >>= 1) d = fmax(d, __shfl_xor(d, o, 64));
+  return d;
+}
+
+// what a thread of k_filter_passes keeps for its passes: LDS offsets of the
+// rows k0-2 .. k0+RB+1 at its column, of the columns a pass and a check read
+// (relative), the nodes it checks and its ghost cell's check
+struct FilterThread {
+  int ro[FILTER_RB + 4], oc[4], os[4], xo[6];
+  unsigned chk, last;   // nodes checked; those on the check's last row
+  bool extra;
+  double Ab, At;        // T: the ghost rows' constants
+  bool lowz, highz;     // the window holds rows that read them
+};
+
+// one pass (and the check before it) at a thread's nodes.  FINITE: every value
+// of the window is finite; otherwise the stretched-grid form's Txx = Trr - Tx*0
+// makes a pass NaN where a value it reads is not.
+template <bool COMP, bool PW2, bool FINITE>
+__device__ __forceinline__ double filter_nodes(const FilterArgs& a, const FilterThread& th, const double* X, double* Y,
+                                               int k0, double cdts, double* yv) {
+  constexpr int RB = FILTER_RB;
+  const int nz = a.nz;
+  double d = 0.0, col[RB + 4];
+#pragma unroll
+  for (int j = 0; j < RB + 4; j++) {
+    double v = X[th.ro[j]];
+    if constexpr (!COMP) {
+      if (th.lowz && k0 + j - 2 < 0) v = th.Ab - v;
+      if (th.highz && k0 + j - 2 > nz) v = th.At - v;
+    }
+    col[j] = v;
   }
-  if ((tid & 63) == 0) {
-    red[0][tid >> 6] = pm;
-    red[1][tid >> 6] = d;
+#pragma unroll
+  for (int r = 0; r < RB; r++) {
+    const double* x = X + th.ro[r + 2];
+    const double e0 = x[th.oc[0]], e1 = x[th.oc[1]], v = col[r + 2], e3 = x[th.oc[2]], e4 = x[th.oc[3]];
+    double srr = a.d2[2] * e0;
+    srr = srr + a.d2[1] * e1;
+    srr = srr + a.d2[0] * v;
+    srr = srr + a.d2[1] * e3;
+    srr = srr + a.d2[2] * e4;
+    double sss = a.d2[2] * col[r];
+    sss = sss + a.d2[1] * col[r + 1];
+    sss = sss + a.d2[0] * v;
+    sss = sss + a.d2[1] * col[r + 3];
+    sss = sss + a.d2[2] * col[r + 4];
+    double Txx = quot<PW2>(srr, a.dr2, a.rdr2), Tzz = quot<PW2>(sss, a.ds2, a.rds2);
+    if constexpr (!FINITE) {
+      Txx = Txx - Txx * 0.0;
+      Tzz = Tzz - Tzz * 0.0;
+    }
+    double y = v + cdts * (Txx + Tzz);
+    const int k = k0 + r;
+    if constexpr (COMP) {
+      if constexpr (FINITE) {
+        y = fmin(fmax(y, 0.0), 1.0);
+      } else {
+        if (y < 0.0) y = 0.0;
+        if (y > 1.0) y = 1.0;
+      }
+    } else {
+      if (k == 0 && a.Tbot == 0) y = a.Tb;
+      if (k == nz) y = a.Tt;
+    }
+    yv[r] = y;
+    if (k <= nz) Y[th.ro[r + 2]] = y;
+    if (th.chk >> r & 1) {
+      // the jumps to the row below, to the right, and across to the row
+      // above; the jump straight up is the next row's jump down, so only the
+      // check's last row takes its own
+      double n1, n2, n4;
+      if constexpr (COMP) {
+        n1 = X[th.ro[r + 1] + th.os[0]];
+        n2 = X[th.ro[r + 1] + th.os[1]];
+        n4 = X[th.ro[r + 3] + th.os[2]];
+      } else {
+        n1 = col[r + 1];
+        n2 = X[th.ro[r + 1] + th.oc[2]];
+        n4 = X[th.ro[r + 3] + th.oc[2]];
+      }
+      d = fmax(d, fmax(fmax(fabs(n1 - v), fabs(n2 - v)), fmax(fabs(e3 - v), fabs(n4 - v))));
+    }
+  }
+  if (th.last) {
+#pragma unroll
+    for (int r = 0; r < RB; r++)
+      if (th.last >> r & 1) d = fmax(d, fabs((COMP ? X[th.ro[r + 3] + th.os[3]] : col[r + 3]) - col[r + 2]));
+  }
+  if constexpr (COMP) {
+    if (th.extra) {
+      const double v = X[th.xo[0]];
+#pragma unroll
+      for (int q = 1; q < 6; q++) d = fmax(d, fabs(X[th.xo[q]] - v));
+    }
+  }
+  return d;
+}
+
+template <bool COMP, bool PW2>
+__global__ void __launch_bounds__(FILTER_THREADS) k_filter_passes(FilterArgs a, FilterLaunch f) {
+  extern __shared__ double fsm[];
+  __shared__ int s_ok[FILTER_KMAX], s_inf;
+  constexpr int RB = FILTER_RB;
+  const int nx = a.nx, nz = a.nz, K = a.K, tid = threadIdx.x, nthr = blockDim.x;
+  const int lane = tid & 63, wave = tid >> 6, nwave = nthr >> 6;
+  const int W = a.pitch, ne = a.pitch * a.rows;
+  double* const dmax = fsm + 2 * ne;   // [K][nthr]: every thread's part of each check
+  if (tid == 0) s_inf = 0;
+  // XCD-aware tiles: workgroups are dealt round-robin over the 8 XCDs; each
+  // XCD gets one contiguous band of tiles, the same in every launch, so that
+  // most of what a tile reads is in its own L2
+  const int ntile = a.ntile, q8 = ntile / 8, r8 = ntile % 8, xcd = blockIdx.x % 8;
+  const int tile = xcd * q8 + min(xcd, r8) + blockIdx.x / 8;
+  const bool edge = COMP && tile >= a.nbx * a.nbz;
+  const int bz = edge ? tile - a.nbx * a.nbz : tile / a.nbx;
+  const int bx = edge ? 0 : tile - bz * a.nbx;
+  const int cz0 = bz * a.ch, cz1 = min(cz0 + a.ch, nz + 1);
+  const int cx0 = edge ? 0 : bx * a.cw, cx1 = edge ? nx + 1 : min(cx0 + a.cw, nx + 1);
+  constexpr int EX = COMP ? 3 : 0;   // the C check reads 5 columns to the side, the pass 2
+  const int S = a.strip;
+  const int xlo = edge ? 0 : max(0, cx0 - 2 * K - EX);
+  const int ncol = edge ? 2 * S : min(nx, cx1 - 1 + 2 * K + EX) - xlo + 1;
+  const int zlo = max(0, cz0 - 2 * K), nrow = min(nz, cz1 - 1 + 2 * K) - zlo + 1;
+  // window: element e = row * ncol + column, threads nthr apart
+  const int er0 = tid / ncol, ec0 = tid - er0 * ncol, dr = nthr / ncol, dc = nthr - dr * ncol;
+  auto load = [&](const double* src) {
+    int er = er0, ec = ec0;
+    bool bad = false;
+    while (er < nrow) {
+      constexpr int FB = 5;
+      double v[FB];
+      int at[FB];
+#pragma unroll
+      for (int u = 0; u < FB; u++) {
+        const int i = edge ? (ec < S ? ec : nx - (2 * S - 1 - ec)) : xlo + ec;
+        v[u] = src[(long)(min(zlo + er, nz) + a.h) * a.p + (i + a.h)];
+        at[u] = er < nrow ? er * W + ec : -1;
+        er += dr;
+        ec += dc;
+        if (ec >= ncol) { ec -= ncol; er++; }
+      }
+#pragma unroll
+      for (int u = 0; u < FB; u++)
+        if (at[u] >= 0) {
+          fsm[at[u]] = v[u];
+          bad |= !(fabs(v[u]) < INFINITY);
+        }
+    }
+    if (bad) s_inf = 1;
+  };
+  // the control word, the previous launch's checks (wavefront t takes check
+  // t) and the window are loaded together, before the decision
+  const int decided = f.ctl[0];
+  double pm[4];
+  const bool mine = f.nprev > 0 && wave < f.kprev;
+#pragma unroll
+  for (int u = 0; u < 4; u++)
+    pm[u] = mine && lane + u * 64 < f.nprev ? f.part_prev[(long)wave * f.nprev + lane + u * 64] : 0.0;
+  load(f.in);
+  if (decided != 0 && decided < f.launch) return;
+  if (f.nprev > 0) {
+    double d = fmax(fmax(pm[0], pm[1]), fmax(pm[2], pm[3]));
+    for (int t = wave; t < f.kprev; t += nwave) {
+      if (t != wave) d = 0.0;
+      for (int b = lane + (t == wave ? 256 : 0); b < f.nprev; b += 64) d = fmax(d, f.part_prev[(long)t * f.nprev + b]);
+      d = wave_max_f64(d);
+      if (lane == 0) s_ok[t] = d < a.delta ? 1 : 0;
+    }
+  }
+  // LDS column of a grid column (mirrored into the grid; clamped where a
+  // thread outside its pass's region asks for a column the window lacks)
+  auto strip_col = [&](int m, bool right) { return right ? max(2 * S - 1 - (nx - m), S) : min(m, S - 1); };
+  auto lcol = [&](int i, bool right) {
+    const int m = mirror(i, nx);
+    return min(max(edge ? strip_col(m, right) : m - xlo, 0), ncol - 1);
+  };
+  auto lrow = [&](int k) { return min(max(mirror(k, nz) - zlo, 0), nrow - 1); };
+  // this thread's nodes: column ic, rows k0 .. k0+RB-1 of the first pass's region
+  const int x1 = edge ? 0 : max(0, cx0 - 2 * (K - 1) - EX), z1 = max(0, cz0 - 2 * (K - 1));
+  const int w1 = edge ? 2 * S : a.w1;
+  const int rb = tid / w1, cc = tid - rb * w1;
+  const int ic = edge ? (cc < S ? cc : nx - (2 * S - 1 - cc)) : x1 + cc, k0 = z1 + rb * RB;
+  const bool live = rb < a.nrb && ic <= nx && k0 <= nz, right = edge && cc >= S;
+  // columns beyond the core (edge tiles: beyond the 6 columns at a wall)
+  const int dx = edge ? max(0, right ? nx - 5 - ic : ic - 5) : max(0, max(cx0 - ic, ic - (cx1 - 1)));
+  const int c0 = edge ? cc : lcol(ic, false);
+  FilterThread th;
+  th.oc[0] = lcol(ic - 2, right) - c0;
+  th.oc[1] = lcol(ic - 1, right) - c0;
+  th.oc[2] = lcol(ic + 1, right) - c0;
+  th.oc[3] = lcol(ic + 2, right) - c0;
+#pragma unroll
+  for (int j = 0; j < RB + 4; j++) th.ro[j] = lrow(k0 + j - 2) * W + c0;
+  th.chk = th.last = 0;
+  if (!edge && live && dx == 0) {
+    // the check's own (row, column) of the node, C: in rows of nx+7 values
+    int kk = k0, ii = ic;
+    const int Q = nx + 7;
+    if constexpr (COMP) {
+      const int L = (k0 + 5) * (Q + 4) + ic + 5;
+      kk = L / Q;
+      ii = L - kk * Q - 3;
+      kk -= 3;
+    }
+#pragma unroll
+    for (int r = 0; r < RB; r++) {
+      const int k = k0 + r;
+      if (k >= cz0 && k < cz1 && kk >= 1 && kk <= nz - 1 && ii >= 0 && ii <= nx - 1) {
+        th.chk |= 1u << r;
+        if (kk == nz - 1) th.last |= 1u << r;
+      }
+      kk++;
+      if constexpr (COMP) {
+        ii += 4;
+        if (ii >= Q - 3) { ii -= Q; kk++; }
+      }
+    }
+  }
+  th.os[0] = th.os[1] = th.os[2] = th.os[3] = 0;
+  if constexpr (COMP) {
+    th.os[0] = lcol(ic + 4, right) - c0;
+    th.os[1] = lcol(ic + 5, right) - c0;
+    th.os[2] = lcol(ic - 3, right) - c0;
+    th.os[3] = lcol(ic - 4, right) - c0;
+  }
+  // one ghost cell's check (C): the ghost rows below a bottom tile's columns,
+  // or the ghost columns of an edge tile's rows
+  th.extra = false;
+#pragma unroll
+  for (int q = 0; q < 6; q++) th.xo[q] = 0;
+  if constexpr (COMP) {
+    if (edge || cz0 == 0) {
+      int col, row;
+      bool cell;
+      if (edge) {
+        const int r0 = bz == 0 ? -5 : cz0, r1 = cz1 == nz + 1 ? nz + 5 : cz1 - 1;
+        const int rr = tid / 10, q = tid - rr * 10;
+        col = q < 5 ? q - 5 : nx + q - 4;
+        row = r0 + rr;
+        cell = row <= r1;
+      } else {
+        const int rr = tid / a.cw;
+        col = cx0 + tid - rr * a.cw;
+        row = -1 - rr;
+        cell = rr < 5 && col < cx1;
+      }
+      if (cell) {
+        const int P = nx + 11, Q = nx + 7, L = (row + 5) * P + col + 5;
+        const int kk = L / Q - 3, ii = L - (kk + 3) * Q - 3;
+        th.extra = kk >= 1 && kk <= nz - 1 && ii >= 0 && ii <= nx - 1;
+        const int nb[6] = {0, -Q, -Q + 1, 1, Q, Q + 1};
+#pragma unroll
+        for (int q = 0; q < 6; q++) {
+          const int Lq = th.extra ? L + nb[q] : 5 * P + 5;
+          const int i = Lq % P - 5;
+          th.xo[q] = lrow(Lq / P - 5) * W + lcol(i, edge && 2 * i >= nx);
+        }
+      }
+    }
+  }
+  // T: the ghost rows' constants
+  th.Ab = th.At = 0.0;
+  th.lowz = th.highz = false;
+  if constexpr (!COMP) {
+    const int i = min(max(ic, 0), nx);
+    const double cb = a.Cvis[(long)5 * (nx + 11) + (i + 5)], ct = a.Cvis[(long)(nz + 5) * (nx + 11) + (i + 5)];
+    th.Ab = 2.0 * a.Tb + a.two_over_d20 * (a.Htype * cb + a.H * (1.0 - (0.0 + cb))) * a.ds2;
+    th.At = 2.0 * a.Tt + a.two_over_d20 * (a.Htype * ct + a.H * (1.0 - (0.0 + ct))) * a.ds2;
+    th.lowz = a.Tbot == 0 && zlo == 0;
+    th.highz = zlo + nrow > nz;
   }
   __syncthreads();
-  if (pass > 1 && fmax(fmax(red[0][0], red[0][1]), fmax(red[0][2], red[0][3])) < delta) {
-    if (bid == 0 && tid == 0) {
-      ctl[1] = pass - 2;   // passes made before the successful check
-      ctl[0] = 1;
+  int np = f.k;           // passes this launch makes
+  bool final = false;
+  if (f.nprev > 0) {
+    int t = 0;
+    while (t < f.kprev && !s_ok[t]) t++;
+    if (t < f.kprev) {
+      final = true;
+      np = t;
+      if (blockIdx.x == 0 && tid == 0) {
+        f.ctl[1] = f.jprev + t;
+        f.ctl[2] = t == 0 ? f.prev_id : f.out_id;
+        f.ctl[0] = f.launch;
+      }
+      if (t == 0 || edge) return;
+      load(f.prev);
+      __syncthreads();
     }
-    return;
   }
-  if (bid < ncheck && tid == 0)
-    sm[(long)cur * SC_BLOCKS + bid] =
-        (unsigned long long)__double_as_longlong(fmax(fmax(red[1][0], red[1][1]), fmax(red[1][2], red[1][3])));
-  if (!node) return;
-  auto W = [&](int u, int v, double val) { out[(long)(v + h) * p + (u + h)] = val; };
-  // the columns whose ghost images equal this node's column: itself, and
-  // its mirror beyond a side wall when it lies within h of that wall
-  int cols[2] = {i, i};
-  int ncol = 1;
-  if (i >= 1 && i <= h) cols[ncol++] = -i;
-  else if (i >= nx - h && i <= nx - 1) cols[ncol++] = 2 * nx - i;
-  if (a.clamp01) {
-    if (y < 0.0) y = 0.0;
-    if (y > 1.0) y = 1.0;
-    for (int c = 0; c < ncol; c++) {
-      W(cols[c], k, y);
-      if (k >= 1 && k <= h) W(cols[c], -k, y);
-      if (k >= nz - h && k <= nz - 1) W(cols[c], 2 * nz - k, y);
+  const bool finite = s_inf == 0;
+  int at0 = 0;
+  double yv[RB];
+#pragma unroll
+  for (int r = 0; r < RB; r++) yv[r] = 0.0;
+  for (int t = 1; t <= np; t++) {
+    const double cdts = final ? f.cdp[t - 1] : f.cd[t - 1];
+    const int left = np - t, hz = 2 * left;
+    const int hx = edge ? 2 * (left - 1) : (left > 0 ? 2 * left + EX : 0);
+    const double* X = fsm + at0;
+    double* Y = fsm + (ne - at0);
+    double d = 0.0;
+    const bool pass = live && dx <= hx && k0 < cz1 + hz && k0 + RB > cz0 - hz;
+    if (pass) {
+      d = finite ? filter_nodes<COMP, PW2, true>(a, th, X, Y, k0, cdts, yv)
+                 : filter_nodes<COMP, PW2, false>(a, th, X, Y, k0, cdts, yv);
+    } else if (COMP && th.extra) {
+      const double v = X[th.xo[0]];
+#pragma unroll
+      for (int q = 1; q < 6; q++) d = fmax(d, fabs(X[th.xo[q]] - v));
     }
-    return;
+    if (!final) dmax[(t - 1) * nthr + tid] = d;
+    __syncthreads();
+    at0 = ne - at0;
   }
-  // T: the wall rows hold the isothermal values (the insulating bottom keeps
-  // its filtered value); ghost rows are 2 T_wall + (2/D2(0)) H ds^2 - mirror
-  // (isothermal) or the mirror (insulating bottom)
-  if (k == 0 && a.Tbot == 0) y = a.Tb;
-  if (k == nz) y = a.Tt;
-  for (int c = 0; c < ncol; c++) {
-    const int col = cols[c];
-    W(col, k, y);
-    if (k >= 1 && k <= h) {
-      const double cb = a.Cvis[(long)5 * (nx + 11) + (col + 5)];
-      const double hb = a.Htype * cb + a.H * (1.0 - (0.0 + cb));
-      W(col, -k, a.Tbot == 0 ? 2.0 * a.Tb + a.two_over_d20 * hb * a.ds2 - y : y);
+  if (!final)
+    for (int t = wave; t < np; t += nwave) {
+      double d = 0.0;
+      for (int u = lane; u < nthr; u += 64) d = fmax(d, dmax[t * nthr + u]);
+      d = wave_max_f64(d);
+      if (lane == 0) f.part[(long)t * ntile + tile] = d;
     }
-    if (k >= nz - h && k <= nz - 1) {
-      const double ct = a.Cvis[(long)(nz + 5) * (nx + 11) + (col + 5)];
-      const double ht = a.Htype * ct + a.H * (1.0 - (0.0 + ct));
-      W(col, 2 * nz - k, 2.0 * a.Tt + a.two_over_d20 * ht * a.ds2 - y);
-    }
+  if (edge || !live || dx > 0) return;
+  // the core's nodes and their ghost images: the columns whose images equal
+  // this node's column are itself and its mirrors beyond the side walls
+  const int h = a.h, p = a.p;
+#pragma unroll
+  for (int r = 0; r < RB; r++) {
+    const int k = k0 + r;
+    if (k < cz0 || k >= cz1) continue;
+    const double y = yv[r];
+    auto column = [&](int c) {
+      auto put = [&](int row, double v) { f.out[(long)(row + h) * p + (c + h)] = v; };
+      put(k, y);
+      if (k >= 1 && k <= h) put(-k, !COMP && a.Tbot == 0 ? th.Ab - y : y);
+      if (k >= nz - h && k <= nz - 1) put(2 * nz - k, COMP ? y : th.At - y);
+    };
+    column(ic);
+    if (ic >= 1 && ic <= h) column(-ic);
+    if (ic >= nx - h && ic <= nx - 1) column(2 * nx - ic);
   }
 }
 
-// one device-driven filter loop on x0 (x1: the second buffer).  cdts_of(j)
-// is pass j's c*dts; on return x0 holds the filtered field with its ghosts
-// and *passes the number of passes made before the successful check
-static int filter_loop(Context& c, double* x0, double* x1, const FilterArgs& fa, double delta,
+// partial maxima of many tiles to one set (grids whose tiles are too many for
+// every tile of the next launch to reduce them itself)
+__global__ void __launch_bounds__(1024) k_filter_reduce(const double* part, int n, double* out) {
+  __shared__ double red[16];
+  const int t = blockIdx.x, tid = threadIdx.x;
+  double d = 0.0;
+  for (int b = tid; b < n; b += 1024) d = fmax(d, part[(long)t * n + b]);
+  d = wave_max_f64(d);
+  if ((tid & 63) == 0) red[tid >> 6] = d;
+  __syncthreads();
+  if (tid == 0) {
+    for (int w = 1; w < 16; w++) d = fmax(d, red[w]);
+    out[t] = d;
+  }
+}
+
+// a tiling's part of the arguments
+static FilterArgs filter_shape(int nx, int nz, bool comp, const FilterPlan& p) {
+  FilterArgs a;
+  const int EX = comp ? 3 : 0;
+  a.nx = nx; a.nz = nz; a.h = comp ? 5 : 3; a.p = nx + 1 + 2 * a.h;
+  a.K = p.K; a.cw = p.cw; a.ch = p.ch;
+  a.nbx = (nx + a.cw) / a.cw; a.nbz = (nz + a.ch) / a.ch;
+  a.strip = std::min(nx + 1, 6 + 2 * (a.K - 1));
+  a.ntile = a.nbx * a.nbz + (comp ? a.nbz : 0);
+  a.pitch = std::min(a.cw + 2 * (2 * a.K + EX), nx + 1);
+  if (comp) a.pitch = std::max(a.pitch, 2 * a.strip);
+  a.rows = std::min(a.ch + 4 * a.K, nz + 1);
+  a.w1 = std::min(a.cw + 2 * (2 * (a.K - 1) + EX), nx + 1);
+  a.nrb = (std::min(a.ch + 4 * (a.K - 1), nz + 1) + FILTER_RB - 1) / FILTER_RB;
+  return a;
+}
+static int filter_threads(const FilterArgs& a, bool comp) {
+  int n = a.w1 * a.nrb;
+  // an edge tile's strips, its ghost cells, a bottom tile's ghost cells
+  if (comp) n = std::max({n, 2 * a.strip * a.nrb, 10 * (a.ch + 10), 5 * a.cw});
+  return (n + 63) & ~63;
+}
+static size_t filter_lds(const FilterArgs& a, int threads) {
+  return sizeof(double) * (2 * (size_t)a.pitch * a.rows + (size_t)a.K * threads);
+}
+
+// Tiles and passes per launch of a grid's filter loops: the tiling with the
+// least modelled time per pass.  A launch costs 8 us (gap, window load, setup,
+// stores), an evaluation 0.22 us and 0.51 ns per node and tile of a CU, fitted
+// to 64x64 (43x4 cores: 2.0 us a pass), 384x128 (32x8: 2.2) and 1024x256
+// (69x17: 2.9); one pass per launch took 3.3, 3.9 and 5.6 us and the gap.
+static FilterPlan filter_plan(int nx, int nz, bool comp) {
+  constexpr int CUS = 256;
+  const int EX = comp ? 3 : 0;
+  FilterPlan best = {8, 4, 1};
+  double best_us = INFINITY;
+  for (int K = 2; K <= FILTER_KMAX; K += 2)
+    for (int ch = 4; ch <= 34; ch++)
+      for (int nbx = 1; nbx <= (nx + 8) / 8; nbx++) {
+        const int cw = (nx + nbx) / nbx;
+        const FilterArgs a = filter_shape(nx, nz, comp, {cw, ch, K});
+        const int threads = filter_threads(a, comp);
+        if (threads > FILTER_THREADS || filter_lds(a, threads) > FILTER_LDS_BYTES) continue;
+        double us = 0.0;
+        for (int h = 0; h < K; h++) {
+          const int w = std::min(cw + 2 * (2 * h + (h ? EX : 0)), nx + 1);
+          const int rows = std::min(ch + 4 * h + FILTER_RB - 1, nz + FILTER_RB);
+          us += 0.22 + 0.51e-3 * w * rows;
+        }
+        us = (8.0 + us * ((a.ntile + CUS - 1) / CUS)) / K;
+        if (us < best_us) {
+          best_us = us;
+          best = {cw, ch, K};
+        }
+      }
+  return best;
+}
+
+static FilterArgs filter_args(const Context& c, bool comp) {
+  FilterArgs a = filter_shape(c.T.nx, c.T.nz, comp, c.filter[comp]);
+  a.dr2 = c.T.dr2; a.ds2 = c.T.ds2; a.rdr2 = 1.0 / c.T.dr2; a.rds2 = 1.0 / c.T.ds2;
+  for (int q = 0; q < 3; q++) a.d2[q] = c.T.D2[3 + q];
+  a.Tbot = c.P.Tbot; a.Tb = c.Tbot_iso; a.Tt = c.Ttop_iso; a.two_over_d20 = 2.0 / c.T.D2[3];
+  a.H = c.P.H; a.Htype = c.P.Htype; a.Cvis = c.Cvis;
+  a.delta = comp ? c.T.delta_C : c.T.delta_T;
+  return a;
+}
+template <bool COMP, bool PW2>
+static int launch_filter(Context& c, const FilterArgs& a, const FilterLaunch& f, int threads, size_t lds) {
+  // set once per process (a thread-safe static initialisation)
+  static const hipError_t attr_rc = hipFuncSetAttribute((const void*)k_filter_passes<COMP, PW2>,
+                               hipFuncAttributeMaxDynamicSharedMemorySize, FILTER_LDS_BYTES);
+  PT_HIP(attr_rc);
+  hipLaunchKernelGGL((k_filter_passes<COMP, PW2>), dim3(a.ntile), dim3(threads), lds, c.stream, a, f);
+  return PT_OK;
+}
+
+__global__ void k_filter_init(int32_t* ctl) {
+  if (threadIdx.x < 4) ctl[threadIdx.x] = 0;
+}
+
+// one device-driven filter loop on x0 (x1, x2: the other buffers).
+// cdts_of(j) is pass j's c*dts; on return x0 holds the filtered field with
+// its ghosts and *passes the number of passes made before the successful check
+static int filter_loop(Context& c, double* x0, double* x1, double* x2, bool comp,
                        double (*cdts_of)(const Context&, int), int* passes, int* hint) {
-  dim3 b16(64, 4);
-  dim3 gflt = grid2(c.T.nx + 1, c.T.nz + 1, b16);
-  unsigned long long* sm = c.d_fsm;
+  const FilterArgs a = filter_args(c, comp);
+  const int threads = filter_threads(a, comp);
+  const size_t lds = filter_lds(a, threads);
+  double* const buf[3] = {x0, x1, x2};
+  double* const parts[2] = {c.d_fpart, c.d_fpart + (size_t)a.ntile * FILTER_KMAX};
+  const bool reduced = a.ntile > FILTER_MAX_PART, pw2 = pow2(a.dr2) && pow2(a.ds2);
   if (c.timing) timer_begin(c, PT_K_FILTER);
-  hipLaunchKernelGGL(k_filter_init, dim3(1), dim3(256), 0, c.stream, c.d_fctl, sm);
+  hipLaunchKernelGGL(k_filter_init, dim3(1), dim3(64), 0, c.stream, c.d_fctl);
   const int cap = 100000;
   // the first batch covers the previous call's pass count (consecutive
-  // projections need similar counts) and the kernel that decides on its
-  // last check; later batches double
-  int j = 0, batch = std::min(std::max(*hint + 3, 8), 1024);
+  // projections need similar counts) and the launch that decides on its last
+  // check; later batches double.  The first launch makes no more passes than
+  // that count's check needs.
+  const int k1 = std::min(a.K, *hint + 1);
+  int n = 0, done = 0, batch = std::min((*hint + 1 - k1 + a.K - 1) / a.K + 2, 1024 / a.K);
+  FilterLaunch f;
+  f.ctl = c.d_fctl;
+  f.k = f.jprev = 0;
   for (;;) {
     for (int b = 0; b < batch; b++) {
-      j++;
-      const double* in = (j & 1) ? x0 : x1;
-      double* out = (j & 1) ? x1 : x0;
-      hipLaunchKernelGGL(k_filter_pass, gflt, b16, 0, c.stream, in, out, fa, c.d_fctl, sm, (j - 1) % FSLOTS,
-                         j % FSLOTS, j, cdts_of(c, j), delta);
+      n++;
+      f.kprev = f.k;
+      f.k = n == 1 ? k1 : a.K;
+      f.jprev = done - f.kprev;
+      f.in = buf[(n - 1) % 3]; f.prev = buf[(n + 1) % 3]; f.out = buf[n % 3];
+      f.part = parts[n % 2]; f.part_prev = reduced ? c.d_fred : parts[(n + 1) % 2];
+      f.nprev = n == 1 ? 0 : reduced ? 1 : a.ntile;
+      f.launch = n; f.out_id = n % 3; f.prev_id = (n + 1) % 3;
+      for (int t = 0; t < FILTER_KMAX; t++) {
+        f.cd[t] = t < f.k ? cdts_of(c, done + t + 1) : 0.0;
+        f.cdp[t] = t < f.kprev ? cdts_of(c, f.jprev + t + 1) : 0.0;
+      }
+      done += f.k;
+      if (comp) PT_TRY(pw2 ? (launch_filter<true, true>(c, a, f, threads, lds)) : (launch_filter<true, false>(c, a, f, threads, lds)));
+      else PT_TRY(pw2 ? (launch_filter<false, true>(c, a, f, threads, lds)) : (launch_filter<false, false>(c, a, f, threads, lds)));
+      if (reduced)
+        hipLaunchKernelGGL(k_filter_reduce, dim3(f.k), dim3(1024), 0, c.stream, f.part, a.ntile, c.d_fred);
     }
-    PT_HIP(hipMemcpyAsync(c.h_fctl, c.d_fctl, 2 * sizeof(int32_t), hipMemcpyDeviceToHost, c.stream));
+    PT_HIP(hipMemcpyAsync(c.h_fctl, c.d_fctl, 3 * sizeof(int32_t), hipMemcpyDeviceToHost, c.stream));
     PT_HIP(hipStreamSynchronize(c.stream));
     if (c.h_fctl[0]) break;
-    if (j > cap) {
+    if (done > cap) {
       set_error("filter did not reach its smoothness threshold in 100000 passes");
       return PT_ERR_INVALID;
     }
-    batch = std::min(2 * batch, 256);
+    batch = std::min(2 * batch, 256 / a.K);
   }
   if (c.timing) timer_end(c, PT_K_FILTER);
   *passes = c.h_fctl[1];
   *hint = *passes;
-  if (*passes & 1) {
-    // the loop ended on the second buffer
-    const size_t bytes = sizeof(double) * (size_t)(c.T.nx + 1 + 2 * fa.h) * (c.T.nz + 1 + 2 * fa.h);
-    PT_HIP(hipMemcpyAsync(x0, x1, bytes, hipMemcpyDeviceToDevice, c.stream));
+  if (c.h_fctl[2] != 0) {
+    const size_t bytes = sizeof(double) * (size_t)(c.T.nx + 1 + 2 * a.h) * (c.T.nz + 1 + 2 * a.h);
+    PT_HIP(hipMemcpyAsync(x0, buf[c.h_fctl[2]], bytes, hipMemcpyDeviceToDevice, c.stream));
   }
   return PT_OK;
-}
-
-static FilterArgs filter_args(const Context& c, int h, int clamp01) {
-  FilterArgs a;
-  a.nx = c.T.nx; a.nz = c.T.nz; a.h = h; a.p = c.T.nx + 1 + 2 * h;
-  a.dr = c.T.dr; a.ds = c.T.ds; a.dr2 = c.T.dr2; a.ds2 = c.T.ds2;
-  for (int q = 0; q < 5; q++) { a.D1[q] = c.T.D1[q + 1]; a.D2[q] = c.T.D2[q + 1]; }
-  a.clamp01 = clamp01;
-  a.Tbot = c.P.Tbot; a.Tb = c.Tbot_iso; a.Tt = c.Ttop_iso; a.two_over_d20 = 2.0 / c.T.D2[3];
-  a.H = c.P.H; a.Htype = c.P.Htype; a.Cvis = c.Cvis;
-  a.check_h = 3; a.check_p = c.T.nx + 7;
-  return a;
 }
 
 // C passes: the first ten with the Chebyshev-ordered steps that damp the
@@ -834,7 +1187,7 @@ static int smoother_time(Context& c) {
   // the halo-3 shape (PS/smoother.f90:79, :602): sequence association makes
   // it read the C storage with the halo-3 row length
   int P = 0;
-  PT_TRY(filter_loop(c, c.Cvis, c.TxS, filter_args(c, 5, 1), c.T.delta_C, cdts_comp, &P, &c.hint_comp));
+  PT_TRY(filter_loop(c, c.Cvis, c.TxS, c.CxS, true, cdts_comp, &P, &c.hint_comp));
   // n_comp counts the outer iterations after the first ten-pass one
   c.n_comp = P < 10 ? 0 : P - 9;
   return PT_OK;
@@ -887,7 +1240,7 @@ static int smoother_time_T(Context& c) {
   if (c.P.RaT == 0.0 || c.P.ivis == 0) return PT_OK;
   if (c.filter_on_device) {
     int P = 0;
-    PT_TRY(filter_loop(c, c.Tvis, c.CxS, filter_args(c, 3, 0), c.T.delta_T, cdts_temp, &P, &c.hint_temp));
+    PT_TRY(filter_loop(c, c.Tvis, c.CxS, c.TxS, false, cdts_temp, &P, &c.hint_temp));
     c.n_temp = P;
     return PT_OK;
   }
@@ -1703,7 +2056,13 @@ int tracers_alloc(Context& c) {
   DALLOC(c.cellsum, sizeof(double) * 27 * (size_t)ncell);
   DALLOC(c.d_flags, sizeof(int32_t) * 4);
   DALLOC(c.d_fctl, sizeof(int32_t) * 4);
-  DALLOC(c.d_fsm, sizeof(unsigned long long) * FSLOTS * SC_BLOCKS);
+  size_t tiles = 0;
+  for (int comp = 0; comp < 2; comp++) {
+    c.filter[comp] = filter_plan(nx, nz, comp != 0);
+    tiles = std::max(tiles, (size_t)filter_args(c, comp != 0).ntile);
+  }
+  DALLOC(c.d_fpart, sizeof(double) * FILTER_KMAX * 2 * tiles);
+  DALLOC(c.d_fred, sizeof(double) * FILTER_KMAX);
   PT_HIP(hipHostMalloc((void**)&c.h_fctl, sizeof(int32_t) * 4, hipHostMallocDefault));
   hipLaunchKernelGGL(k_iota, dim3((unsigned)((c.T.ntr + 255) / 256)), dim3(256), 0, 0, c.iota, c.T.ntr);
   c.sort_bits = 1;
@@ -1718,7 +2077,7 @@ int tracers_free(Context& c) {
   void* ps[] = {c.SF, c.Tratio, c.T0, c.Tvis, c.Tbuoy, c.u, c.w, c.src, c.cond_r, c.cond_s, c.Cnew, c.C0, c.Cvis,
                 c.Cbuoy, c.cond, c.Textend, c.TxS, c.CxS, c.itab, c.ctab, c.dtab, c.r, c.s, c.Tt, c.Ct, c.r0, c.s0, c.T0t,
                 c.r1, c.s1, c.T1t, c.r2, c.s2, c.T2t, c.cellkey, c.skey, c.iota, c.perm, c.tid, c.tid_tmp, c.cstart, c.cend,
-                c.nempty, c.cellsum, c.d_flags, c.sort_tmp, c.d_fctl, c.d_fsm, c.okey, c.ostart, c.oend, c.ccount,
+                c.nempty, c.cellsum, c.d_flags, c.sort_tmp, c.d_fctl, c.d_fpart, c.d_fred, c.okey, c.ostart, c.oend, c.ccount,
                 c.bsum};
   for (void* p : ps)
     if (p) (void)hipFree(p);
