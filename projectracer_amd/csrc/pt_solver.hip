@@ -1324,6 +1324,13 @@ static SweepPlan sweep_plan(const Context& c, int l, bool f32, int s) {
           if (base + (rem ? 1 : 0) != ns) continue;   // a larger ns with as many launches
           const SweepShape widest = sweep_shape(n, m, cw, ch, rb, ns + extra, elem);
           if (widest.threads > sweep_threads_of(f32, ev, rb) || widest.lds > SWEEP_LDS_BYTES) break;
+          // not the tilings whose tiles mostly recompute each other's points, nor
+          // those of several points per thread in few wavefronts: the model does
+          // not hold there
+          double evals = 0.0;
+          for (int h = 0; h < ns; h++) evals += (double)std::min(cw + 6 * h, n - 1) * std::min(ch + 6 * h, m - 1);
+          if (widest.nblk > 1 && evals * widest.nblk > (nseg == 1 ? 2.0 : 5.0) * ns * (n - 1) * (m - 1)) continue;
+          if (rb > 1 && widest.threads < 512) continue;
           double us = rem * sweep_launch_us(cost, n, m, cw, ch, rb, ns, sweep_shape(n, m, cw, ch, rb, ns, elem));
           if (nseg > rem + 1)
             us += (nseg - rem - 1) *
