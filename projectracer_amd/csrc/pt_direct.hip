@@ -8,12 +8,13 @@
 // solution into psi with its ghost images (Stream_grid).
 //
 // Device layout: AB column-major, A(p,q) at AB[(q-1)*LDAB + kl+ku+p-q]; the
-// factorization is one workgroup of 1024 threads walking the columns; the
-// solve is one workgroup whose band window lives in an LDS ring.
+// factorization walks the columns in panels, a wavefront per column; the solve
+// is one workgroup whose band window lives in an LDS ring.
 #include "pt_internal.hpp"
 
 #include <algorithm>
 #include <cstring>
+#include <type_traits>
 
 namespace pt {
 
@@ -154,157 +155,249 @@ __global__ void k_sf_assemble(SfArgs a, const double* vis, double* ab) {
 
 // ---------------------------------------------------------------------------
 // DGBTF2 (band LU with partial pivoting, LAPACK's unblocked column order) in
-// panels of nb columns.
-//   k_lu_panel: one workgroup factors columns p0 .. p0+nb-1 held in LDS
-//     (rows p0 .. p0+nb-1+kl): per column the first-maximum pivot search, the
-//     row interchange, the scaling and the rank-1 update, each restricted to
-//     the panel's columns.  It records ju after every step (the last column
-//     DGBTF2's step touches; -1 for a zero pivot, which DGBTF2 skips).
-//   k_lu_trailing: one wave per column beyond the panel replays the panel's
-//     steps on that column in order -- the interchange, then
-//     x = x + L(t,j) (-A(j,c)) -- while the column is within the step's ju.
+// panels of LU_NB columns, each column held by a wavefront in registers.
+//   k_lu_panel: one workgroup factors columns p0 .. p0+LU_NB-1, a wavefront
+//     per column.  At step s the columns behind it apply the step (interchange,
+//     rank-1 update); the wavefront of column s+1 then finds its pivot (DPP
+//     maxima), scales the multipliers and leaves them in LDS.  One barrier per
+//     step.  It records ju after every step (the last column DGBTF2's step
+//     touches; -1 for a zero pivot, which DGBTF2 skips).
+//   k_lu_trailing: a wavefront per column beyond the panel replays the panel's
+//     steps on it in order -- the interchange, then x = x + L(t,j) (-A(j,c)) --
+//     while the column is within the step's ju.
 // Every element sees the operations of DGBTF2 in the same order, so the
 // factors are DGBTF2's bit for bit.  AB's fill rows start zero (memset) and
 // are first written by the step that DGBTF2 zeroes them at, so that zeroing
 // is not repeated.
+// Bound by the chain of steps: apply to the next column, pivot search, scaling,
+// barrier, one compute unit at work.  100x100 (n = 10201, kl = 303), build in
+// all: 38.6 ms with a thread per row, the panel in LDS and three barriers per
+// column (panel of 32: 100 us; trailing columns in LDS 25 us); 14.5 ms now
+// (panel of 16: 14.2 us, trailing 8.0 us).  With rows per thread and the panel
+// in registers every column's pivot row passes through LDS, in any form of it
+// 1.6 us a step: 22 ms.  Panels of 32 (two columns per wavefront) 18.6 ms, of
+// 24 19.6, of 8 19.4 (these three with more registers than now).
 // ---------------------------------------------------------------------------
-constexpr int LU_PANEL_THREADS = 1024;   // upper bound; launched with roundup64(kl+1) threads
+constexpr int LU_NB = 16;                         // panel columns: the wavefronts of a workgroup
+constexpr int LU_MAX_KL = 1023;                   // at most 17 rows per lane
 constexpr int LU_LDS_LIMIT = 160 * 1024 - 1024;   // dynamic LDS per workgroup (gfx950: 160 KB)
-constexpr int LU_TRAIL_WAVES = 8;   // columns per trailing workgroup
+constexpr int LU_TRAIL_WAVES = 8;                 // columns per trailing workgroup
 
-__global__ void __launch_bounds__(LU_PANEL_THREADS) k_lu_panel(double* ab, int32_t* ipiv, int32_t* ju_rec,
-                                                               int32_t* state, int n, int kl, int ku, int p0,
-                                                               int nb) {
-  extern __shared__ double P[];   // P[(c-p0)*W + (r-p0)], W = kl + nb
-  __shared__ double s_best[LU_PANEL_THREADS / 64];
-  __shared__ int s_idx[LU_PANEL_THREADS / 64];
-  __shared__ int s_jp;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, NT = blockDim.x, nwv = NT >> 6;
+// the value of v in lane `lane` (uniform), as a uniform double
+__device__ __forceinline__ double readlane_f64(double v, int lane) {
+  const long long x = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_readlane((int)(x & 0xffffffffLL), lane);
+  const int hi = __builtin_amdgcn_readlane((int)(x >> 32), lane);
+  return __longlong_as_double(((long long)hi << 32) | (long long)(unsigned int)lo);
+}
+
+// one DPP step of a maximum of unsigned words over lanes (0 where the step has
+// no source lane): a single instruction, where doubles would need two moves
+// and two maxima
+template <int CTRL, int ROWS>
+__device__ __forceinline__ unsigned max_dpp(unsigned v) {
+  return max(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROWS, 0xf, false));
+}
+// maxima of each row of 16 lanes, in its lane 15 (row_shr 1, 2, 4, 8)
+__device__ __forceinline__ unsigned row_max_dpp(unsigned v) {
+  return max_dpp<0x118, 0xf>(max_dpp<0x114, 0xf>(max_dpp<0x112, 0xf>(max_dpp<0x111, 0xf>(v))));
+}
+// maximum over the wavefront, as a uniform value (row_bcast 15, 31)
+__device__ __forceinline__ unsigned wave_max_dpp(unsigned v) {
+  return __builtin_amdgcn_readlane(max_dpp<0x143, 0xc>(max_dpp<0x142, 0xa>(row_max_dpp(v))), 63);
+}
+
+// A wavefront holds a column of the panel's rows in registers: row 64 q + lane
+// in x[q].
+
+// rows s and l of the column change places; returns the new row s.  (No branch
+// on the register of row l: where the paths meet, the column would be copied.)
+template <int Q>
+__device__ __forceinline__ double lu_swap(double (&x)[Q], int s, int l, int lane) {
+  const double top = readlane_f64(x[0], s);
+  double t = x[0];
+#pragma unroll
+  for (int q = 0; q < Q; q++) {
+    const bool here = 64 * q + lane == l;
+    t = here ? x[q] : t;
+    x[q] = here ? top : x[q];
+  }
+  const double low = readlane_f64(t, l & 63);
+  x[0] = lane == s ? low : x[0];
+  return low;
+}
+
+// step s of the panel: the interchange, then x = x + L (-x(s)) on rows s+1 .. last
+template <int Q>
+__device__ __forceinline__ void lu_apply(double (&x)[Q], const double (&L)[Q], int s, int l, int last, int lane) {
+  if (l != s) lu_swap(x, s, l, lane);
+  const double temp = -1.0 * readlane_f64(x[0], s);
+#pragma unroll
+  for (int q = 0; q < Q; q++) {
+    const double y = x[q] + L[q] * temp;
+    const int r = 64 * q + lane;
+    x[q] = (q > 0 || r > s) && r <= last ? y : x[q];
+  }
+}
+
+struct LuStep { int l, ju, taken, inf; };   // the step's pivot row, and ju and inf after it
+
+// step s's own column: pivot search, interchange, multipliers
+template <int Q>
+__device__ __forceinline__ LuStep lu_pivot(double (&x)[Q], double* Ls, int s, int col, int last, int ku, int n, int ju,
+                                           int inf, int lane) {
+  // the first of the rows with the largest entry that is a number
+  double v = -1.0;
+  int row = 0;
+#pragma unroll
+  for (int q = 0; q < Q; q++) {
+    const double y = fabs(x[q]);
+    const int r = 64 * q + lane;
+    if ((q > 0 || r >= s) && r <= last && y > v) { v = y; row = r; }
+  }
+  // over the lanes, magnitudes compare as integers: the high words decide but
+  // for ties (DPP maxima of single words, no LDS)
+  const unsigned long long key = (unsigned long long)__double_as_longlong(v);
+  const unsigned kh = v >= 0.0 ? (unsigned)(key >> 32) + 1u : 0u, hm = wave_max_dpp(kh);
+  unsigned long long at = __ballot(kh == hm);
+  int l = __builtin_amdgcn_readlane(row, __ffsll((long long)at) - 1);
+  if (at & (at - 1)) {
+    const unsigned kw = kh == hm ? (unsigned)key : 0u, wm = wave_max_dpp(kw);
+    l = ~(int)wave_max_dpp(kh == hm && kw == wm ? ~(unsigned)row : 0u);
+  }
+  if (hm == 0u) l = s;   // no candidate is a number
+  const double piv = l != s ? lu_swap(x, s, l, lane) : readlane_f64(x[0], s);
+  LuStep st{l, ju, piv != 0.0, inf};
+  if (st.taken) {
+    st.ju = max(ju, min(col + ku + (l - s), n));
+    const double rcp = 1.0 / piv;
+#pragma unroll
+    for (int q = 0; q < Q; q++) {
+      const double y = rcp * x[q];
+      const int r = 64 * q + lane;
+      x[q] = (q > 0 || r > s) && r <= last ? y : x[q];
+      Ls[r] = x[q];
+    }
+  } else if (inf == 0) {
+    st.inf = col;
+  }
+  return st;
+}
+
+template <int Q>   // rows per lane
+__global__ void __launch_bounds__(LU_NB * 64) k_lu_panel(double* ab, int32_t* ipiv, int32_t* ju_rec, int32_t* state,
+                                                         int n, int kl, int ku, int p0) {
+  __shared__ double Ls[2][64 * Q];   // the step's multipliers
+  __shared__ LuStep step[2];
+  const int lane = threadIdx.x & 63, c = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const long ld = 2 * kl + ku + 1;
-  const int kv = ku + kl, W = kl + nb, pe = min(p0 + nb - 1, n), np = pe - p0 + 1;
-  // A(r, c) = AB(kv+1+r-c, c): rows above c+kl are stored for c >= p0
-  for (int e = tid; e < np * W; e += NT) {
-    const int cc = e / W, r = e - cc * W, col = p0 + cc, row = p0 + r;
-    P[e] = (row <= min(n, col + kl)) ? ab[(long)(col - 1) * ld + (kv + row - col)] : 0.0;
+  const int kv = ku + kl, np = min(LU_NB, n - p0 + 1);
+  // the wavefront's column: rows p0 .. p0+kl+LU_NB-1 that are stored
+  const int lo = c - kv, hi = min(n - p0, c + kl);
+  double x[Q];
+#pragma unroll
+  for (int q = 0; q < Q; q++) {
+    const int r = 64 * q + lane;
+    x[q] = c < np && r >= lo && r <= hi ? ab[(long)(p0 + c - 1) * ld + (kv + r - c)] : 0.0;
   }
+  auto pivot = [&](int ju, int inf) {
+    const int col = p0 + c;
+    const LuStep st = lu_pivot(x, Ls[c & 1], c, col, c + min(kl, n - col), ku, n, ju, inf, lane);
+    if (lane == 0) {
+      step[c & 1] = st;
+      ipiv[col - 1] = p0 + st.l;
+      ju_rec[col - 1] = st.taken ? st.ju : -1;
+    }
+  };
   // ju and the first zero pivot carried between panels
-  int ju = (p0 == 1) ? 1 : state[0];
-  int inf = (p0 == 1) ? 0 : state[1];
-  __syncthreads();
-  auto A = [&](int r, int col) -> double& { return P[(col - p0) * W + (r - p0)]; };
-  for (int j = p0; j <= pe; j++) {
-    const int km = min(kl, n - j);
-    double best = -1.0;
-    int bi = 0x7fffffff;
-    for (int t = tid; t <= km; t += NT) {
-      const double x = fabs(A(j + t, j));
-      if (x > best) { best = x; bi = t; }
-    }
-    for (int off = 32; off > 0; off >>= 1) {
-      const double ob = __shfl_down(best, off);
-      const int oi = __shfl_down(bi, off);
-      if (ob > best || (ob == best && oi < bi)) { best = ob; bi = oi; }
-    }
-    if (lane == 0) { s_best[wave] = best; s_idx[wave] = bi; }
+  if (c == 0) pivot(p0 == 1 ? 1 : state[0], p0 == 1 ? 0 : state[1]);
+  for (int s = 0; s < np; s++) {
     __syncthreads();
-    if (tid == 0) {
-      double b = s_best[0];
-      int x = s_idx[0];
-      for (int w = 1; w < nwv; w++)
-        if (s_best[w] > b || (s_best[w] == b && s_idx[w] < x)) { b = s_best[w]; x = s_idx[w]; }
-      s_jp = x + 1;
-      ipiv[j - 1] = x + j;
+    const LuStep st = step[s & 1];
+    const int l = __builtin_amdgcn_readfirstlane(st.l), ju = __builtin_amdgcn_readfirstlane(st.ju);
+    const int taken = __builtin_amdgcn_readfirstlane(st.taken), inf = __builtin_amdgcn_readfirstlane(st.inf);
+    if (s + 1 == np) {
+      if (threadIdx.x == 0) { state[0] = ju; state[1] = inf; }
+      break;
     }
-    __syncthreads();
-    const int jp = s_jp;
-    if (A(j + jp - 1, j) != 0.0) {
-      ju = max(ju, min(j + ku + jp - 1, n));
-      const int ce = min(ju, pe);
-      if (jp != 1)
-        for (int col = j + tid; col <= ce; col += NT) {
-          const double tmp = A(j + jp - 1, col);
-          A(j + jp - 1, col) = A(j, col);
-          A(j, col) = tmp;
-        }
-      __syncthreads();
-      if (km > 0) {
-        // thread t owns row j+1+t of the panel (km <= kl < blockDim): the
-        // scaled multiplier stays in a register for the rank-1 update
-        const double rcp = 1.0 / A(j, j);
-        const int t = 1 + tid;
-        double lt = 0.0;
-        if (t <= km) {
-          lt = rcp * A(j + t, j);
-          A(j + t, j) = lt;
-        }
-#pragma unroll 8
-        for (int col = j + 1; col <= ce; col++) {
-          const double temp = -1.0 * A(j, col);
-          if (t <= km) A(j + t, col) = A(j + t, col) + lt * temp;
-        }
-      }
-      if (tid == 0) ju_rec[j - 1] = ju;
-    } else {
-      if (inf == 0) inf = j;
-      if (tid == 0) ju_rec[j - 1] = -1;
-    }
-    __syncthreads();
+    if (c <= s || c >= np) continue;
+    double L[Q];
+#pragma unroll
+    for (int q = 0; q < Q; q++) L[q] = Ls[s & 1][64 * q + lane];
+    if (taken && p0 + c <= ju) lu_apply(x, L, s, l, s + min(kl, n - (p0 + s)), lane);
+    if (c == s + 1) pivot(ju, inf);
   }
-  for (int e = tid; e < np * W; e += NT) {
-    const int cc = e / W, r = e - cc * W, col = p0 + cc, row = p0 + r;
-    if (row <= min(n, col + kl)) ab[(long)(col - 1) * ld + (kv + row - col)] = P[e];
+  // (the loads' addresses are not kept through the loop: they would take as
+  // many registers as the column)
+  int row0 = lane;
+  asm volatile("" : "+v"(row0));
+#pragma unroll
+  for (int q = 0; q < Q; q++) {
+    const int r = 64 * q + row0;
+    if (c < np && r >= lo && r <= hi) ab[(long)(p0 + c - 1) * ld + (kv + r - c)] = x[q];
   }
-  if (tid == 0) { state[0] = ju; state[1] = inf; }
 }
 
-// wave-level ordering of LDS accesses between lanes of one wave
-__device__ __forceinline__ void wave_lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
+template <int Q>   // rows per lane
 __global__ void __launch_bounds__(LU_TRAIL_WAVES * 64) k_lu_trailing(double* ab, const int32_t* ipiv,
                                                                      const int32_t* ju_rec, int n, int kl, int ku,
-                                                                     int p0, int nb) {
-  extern __shared__ double sh[];
+                                                                     int p0) {
+  extern __shared__ double Ls[];   // Ls[s*W + r] = L(p0+r, p0+s)
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const long ld = 2 * kl + ku + 1;
-  const int kv = ku + kl, W = kl + nb, pe = min(p0 + nb - 1, n), np = pe - p0 + 1;
-  double* Ls = sh;                                   // Ls[s*kl + t-1] = L(p0+s+t, p0+s)
-  double* Cb = sh + (size_t)nb * kl + (size_t)wave * W;   // this wave's column, rows p0 .. p0+W-1
-  for (int e = tid; e < np * kl; e += LU_TRAIL_WAVES * 64) {
-    const int sc = e / kl, t = 1 + (e - sc * kl), j = p0 + sc;
-    Ls[e] = (t <= min(kl, n - j)) ? ab[(long)(j - 1) * ld + (kv + t)] : 0.0;
+  const int kv = ku + kl, W = kl + LU_NB, pe = min(p0 + LU_NB - 1, n), np = pe - p0 + 1;
+  const int c = pe + 1 + blockIdx.x * LU_TRAIL_WAVES + wave;
+  const bool live = c <= min(n, pe + kv);
+  // this wavefront's column: rows p0 .. p0+W-1 that are stored
+  const int lo = c - kv - p0, hi = min(n, c + kl) - p0;
+  double x[Q];
+#pragma unroll
+  for (int q = 0; q < Q; q++) {
+    const int r = 64 * q + lane;
+    x[q] = live && r < W && r >= lo && r <= hi ? ab[(long)(c - 1) * ld + (kv + p0 + r - c)] : 0.0;
+  }
+  // the panel's multipliers (entries that are none are read from a stored
+  // place and not used), and each step's ju and interchange in lane s
+  const int js = p0 + min(lane, np - 1);
+  const int juv = ju_rec[js - 1], lv = ipiv[js - 1] - p0;
+  static_assert(LU_NB == 2 * LU_TRAIL_WAVES, "two of the panel's columns per wavefront");
+  double v[2][Q];
+#pragma unroll
+  for (int u = 0; u < 2; u++) {
+    const int sc = min(wave + u * LU_TRAIL_WAVES, np - 1);
+#pragma unroll
+    for (int q = 0; q < Q; q++)
+      v[u][q] = ab[(long)(p0 + sc - 1) * ld + (kv + min(max(64 * q + lane - sc, 0), kl))];
+  }
+#pragma unroll
+  for (int u = 0; u < 2; u++) {
+    const int sc = wave + u * LU_TRAIL_WAVES;
+#pragma unroll
+    for (int q = 0; q < Q; q++)
+      if (sc < np && 64 * q + lane < W) Ls[sc * W + 64 * q + lane] = v[u][q];
   }
   __syncthreads();
-  const int c = pe + 1 + blockIdx.x * LU_TRAIL_WAVES + wave;
-  if (c > min(n, pe + kv)) return;
-  for (int r = lane; r < W; r += 64) {
-    const int row = p0 + r;
-    Cb[r] = (row >= c - kv && row <= min(n, c + kl)) ? ab[(long)(c - 1) * ld + (kv + row - c)] : 0.0;
-  }
-  wave_lds_sync();
+  if (!live) return;
+  double L[Q];
+  auto fetch = [&](int sc) {
+#pragma unroll
+    for (int q = 0; q < Q; q++) L[q] = Ls[sc * W + min(64 * q + lane, W - 1)];
+  };
+  fetch(0);
   for (int sc = 0; sc < np; sc++) {
-    const int j = p0 + sc, jut = ju_rec[j - 1];
+    double Lc[Q];
+#pragma unroll
+    for (int q = 0; q < Q; q++) Lc[q] = L[q];
+    fetch(min(sc + 1, np - 1));   // the next step's multipliers
+    const int j = p0 + sc, jut = __builtin_amdgcn_readlane(juv, sc);
     if (jut < 0 || c > jut) continue;
-    const int l = ipiv[j - 1];
-    if (l != j) {
-      if (lane == 0) {
-        const double tmp = Cb[l - p0];
-        Cb[l - p0] = Cb[sc];
-        Cb[sc] = tmp;
-      }
-      wave_lds_sync();
-    }
-    const double temp = -1.0 * Cb[sc];
-    const int km = min(kl, n - j);
-    for (int t = 1 + lane; t <= km; t += 64) Cb[sc + t] = Cb[sc + t] + Ls[sc * kl + t - 1] * temp;
-    wave_lds_sync();
+    const int l = __builtin_amdgcn_readlane(lv, sc), last = sc + min(kl, n - j);
+    lu_apply(x, Lc, sc, l, last, lane);
   }
-  for (int r = lane; r < W; r += 64) {
-    const int row = p0 + r;
-    if (row >= c - kv && row <= min(n, c + kl)) ab[(long)(c - 1) * ld + (kv + row - c)] = Cb[r];
+#pragma unroll
+  for (int q = 0; q < Q; q++) {
+    const int r = 64 * q + lane;
+    if (r < W && r >= lo && r <= hi) ab[(long)(c - 1) * ld + (kv + p0 + r - c)] = x[q];
   }
 }
 
@@ -335,14 +428,6 @@ constexpr int CHUNK = 512;
 constexpr int NBH = 64;   // head rows per block: one wavefront
 
 __device__ __forceinline__ int ring_slot(int pos) { return (pos - 1) & (RING - 1); }
-
-// the value of v in lane `lane` (uniform), as a uniform double
-__device__ __forceinline__ double readlane_f64(double v, int lane) {
-  const long long x = __double_as_longlong(v);
-  const int lo = __builtin_amdgcn_readlane((int)(x & 0xffffffffLL), lane);
-  const int hi = __builtin_amdgcn_readlane((int)(x >> 32), lane);
-  return __longlong_as_double(((long long)hi << 32) | (long long)(unsigned int)lo);
-}
 
 // forward: L y = P b, in place on b
 template <int E>   // tail rows per thread
@@ -694,41 +779,38 @@ int build_sf_matrix(Context& c) {
   PT_HIP(hipMemsetAsync(c.dAB, 0, sizeof(double) * ld * (size_t)t.dn, c.stream));
   hipLaunchKernelGGL(k_sf_assemble, dim3((t.dn + 127) / 128), dim3(128), 0, c.stream, a, L1.v.vis, c.dAB);
   PT_TRY(launch_equilibrate(c, c.dAB, c.dRow, t.dn, t.dkl, t.dku));
-  // panels of nb columns: the panel in LDS (W = kl+nb rows), the trailing
-  // workgroups hold the panel's L columns and one column per wave
-  int nb = 32;
-  auto panel_lds = [&](int b) { return sizeof(double) * (size_t)(t.dkl + b) * b; };
-  auto trail_lds = [&](int b) { return sizeof(double) * ((size_t)b * t.dkl + (size_t)LU_TRAIL_WAVES * (t.dkl + b)); };
-  while (nb > 4 && (panel_lds(nb) > LU_LDS_LIMIT || trail_lds(nb) > LU_LDS_LIMIT)) nb /= 2;
-  if (panel_lds(nb) > LU_LDS_LIMIT || trail_lds(nb) > LU_LDS_LIMIT) {
-    set_error("direct solver: lower band width too large for the LU panels");
+  if (t.dkl > LU_MAX_KL) {
+    set_error("direct solver: lower band width above " + std::to_string(LU_MAX_KL));
     return PT_ERR_UNSUPPORTED;
   }
-  // set once per process (a thread-safe static initialisation)
-  static const hipError_t attr_rc = [] {
-    const hipError_t e = hipFuncSetAttribute((const void*)k_lu_panel, hipFuncAttributeMaxDynamicSharedMemorySize, LU_LDS_LIMIT);
-    return e != hipSuccess ? e : hipFuncSetAttribute((const void*)k_lu_trailing, hipFuncAttributeMaxDynamicSharedMemorySize,
-                               LU_LDS_LIMIT);
-  }();
-  PT_HIP(attr_rc);
-  const int kv = t.dkl + t.dku;
-  // one thread per subdiagonal row of the pivot column (the panel keeps each
-  // row's multiplier in a register)
-  const int panel_threads = ((t.dkl + 1 + 63) / 64) * 64;
-  if (panel_threads > LU_PANEL_THREADS) {
-    set_error("direct solver: lower band width above " + std::to_string(LU_PANEL_THREADS - 1));
-    return PT_ERR_UNSUPPORTED;
-  }
-  for (int p0 = 1; p0 <= t.dn; p0 += nb) {
-    const int pe = std::min(p0 + nb - 1, t.dn);
-    hipLaunchKernelGGL(k_lu_panel, dim3(1), dim3(panel_threads), panel_lds(nb), c.stream, c.dAB, c.dipiv, c.dju,
-                       c.d_lustate, t.dn, t.dkl, t.dku, p0, nb);
-    const int ncols = std::min(t.dn, pe + kv) - pe;
-    if (ncols > 0)
-      hipLaunchKernelGGL(k_lu_trailing, dim3((ncols + LU_TRAIL_WAVES - 1) / LU_TRAIL_WAVES),
-                         dim3(LU_TRAIL_WAVES * 64), trail_lds(nb), c.stream, c.dAB, c.dipiv, c.dju, t.dn, t.dkl,
-                         t.dku, p0, nb);
-  }
+  const int rows = t.dkl + LU_NB, kv = t.dkl + t.dku;
+  auto factor = [&](auto qc) -> int {
+    constexpr int Q = decltype(qc)::value;
+    // set once per process (a thread-safe static initialisation)
+    static const hipError_t attr_rc = hipFuncSetAttribute(
+        (const void*)k_lu_trailing<Q>, hipFuncAttributeMaxDynamicSharedMemorySize, LU_LDS_LIMIT);
+    PT_HIP(attr_rc);
+    for (int p0 = 1; p0 <= t.dn; p0 += LU_NB) {
+      hipLaunchKernelGGL(k_lu_panel<Q>, dim3(1), dim3(LU_NB * 64), 0, c.stream, c.dAB, c.dipiv, c.dju, c.d_lustate,
+                         t.dn, t.dkl, t.dku, p0);
+      const int pe = std::min(p0 + LU_NB - 1, t.dn), ncols = std::min(t.dn, pe + kv) - pe;
+      if (ncols <= 0) continue;
+      hipLaunchKernelGGL(k_lu_trailing<Q>, dim3((ncols + LU_TRAIL_WAVES - 1) / LU_TRAIL_WAVES),
+                         dim3(LU_TRAIL_WAVES * 64), sizeof(double) * LU_NB * rows, c.stream, c.dAB, c.dipiv, c.dju,
+                         t.dn, t.dkl, t.dku, p0);
+    }
+    return PT_OK;
+  };
+  // rows per lane: the band's height in registers, as little padded as these sizes allow
+  if (rows <= 128) PT_TRY(factor(std::integral_constant<int, 2>{}));
+  else if (rows <= 192) PT_TRY(factor(std::integral_constant<int, 3>{}));
+  else if (rows <= 256) PT_TRY(factor(std::integral_constant<int, 4>{}));
+  else if (rows <= 320) PT_TRY(factor(std::integral_constant<int, 5>{}));
+  else if (rows <= 384) PT_TRY(factor(std::integral_constant<int, 6>{}));
+  else if (rows <= 512) PT_TRY(factor(std::integral_constant<int, 8>{}));
+  else if (rows <= 640) PT_TRY(factor(std::integral_constant<int, 10>{}));
+  else if (rows <= 832) PT_TRY(factor(std::integral_constant<int, 13>{}));
+  else PT_TRY(factor(std::integral_constant<int, 17>{}));
   int32_t info = 0;
   PT_HIP(hipMemcpyAsync(&info, c.d_lustate + 1, sizeof(int32_t), hipMemcpyDeviceToHost, c.stream));
   PT_HIP(hipStreamSynchronize(c.stream));
