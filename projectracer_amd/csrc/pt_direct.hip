@@ -407,11 +407,13 @@ __global__ void __launch_bounds__(LU_TRAIL_WAVES * 64) k_lu_trailing(double* ab,
 // ring (slot = (position-1) mod RING) refilled from global memory in chunks,
 // and finished positions are written back in place.  The column steps are
 // taken NBH (one wavefront) at a time:
-//   head: one wave runs the block's steps on the block's NBH rows, one row
-//     per lane, with the step's value broadcast by v_readlane and the
-//     block's triangle of L (or U) staged in LDS: no barrier per step;
-//   tail: every thread then applies the block's steps to one of the kl (or
-//     kl+ku) rows below (above) the head, in step order.
+//   head: wavefront 0 runs the block's steps on the block's NBH rows, one row
+//     per lane and the block's triangle of L (or U) in registers, with the
+//     step's value broadcast by v_readlane: no barrier per step;
+//   tail: the other wavefronts then apply the block's steps to the kl (or
+//     kl+ku) rows below (above) the head, E rows per thread, in step order.
+// Either loads a block's band entries into registers while the other is at
+// work: the head its next triangle, the tail its next D column steps.
 // Each element sees the same operations in the same order as DGBTRS's
 // column-by-column loops, so the results are identical.  Forward blocks
 // end early where a pivot row would leave the head (the block's first step
@@ -421,256 +423,320 @@ __global__ void __launch_bounds__(LU_TRAIL_WAVES * 64) k_lu_trailing(double* ab,
 //     b(j+1 .. j+kl) += L(., j) (-b(j));
 //   backward (DTBSV, upper, bandwidth kl+ku): x(j) = b(j)/U(j,j) unless b(j)
 //     is zero, then b(j-1 .. j-kl-ku) -= x(j) U(., j).
+// Bound by the chain of a block (head 1.7 us forward, 3.5 us backward with its
+// quotients; then the tail) and by what one compute unit draws from memory,
+// about 40 GB/s.  At 100x100 (160 blocks, bands 303 and 606) forward and
+// backward took 1.73 and 3.56 ms with the loads between the barriers, masked
+// steps and divisions, and take 0.78 and 1.39 ms.  (Reloading each register
+// right after its step would use the tail's time too, but the compiler gives
+// such a loop twice the registers.)
 // ---------------------------------------------------------------------------
-constexpr int SOLVE_MAX_THREADS = 1024;
+constexpr int SOLVE_MAX_TAIL = 640;   // tail threads: 11 wavefronts leave 168 registers each
 constexpr int RING = 4096;
 constexpr int CHUNK = 512;
 constexpr int NBH = 64;   // head rows per block: one wavefront
 
 __device__ __forceinline__ int ring_slot(int pos) { return (pos - 1) & (RING - 1); }
 
-// forward: L y = P b, in place on b
-template <int E>   // tail rows per thread
-__global__ void __launch_bounds__(SOLVE_MAX_THREADS) k_band_forward(const double* __restrict__ ab,
-                                                                    const int32_t* __restrict__ ipiv, double* b,
-                                                                    int n, int kl, int ku) {
-  __shared__ double R[RING];
-  __shared__ double Lh[NBH][NBH];   // Lh[s][r] = L(j0+r, j0+s)
-  __shared__ double T[NBH];         // -b(j) of the block's steps
-  const int tid = threadIdx.x, NT = blockDim.x, lane = tid & 63;
-  const long ld = 2 * kl + ku + 1;
-  const int kd = ku + kl + 1;   // L(j+t, j) = AB(kd+t, j), t = 1..kl (1-based)
-  if (kl == 0 || n < 2) return;
-  auto Lg = [&](int r, int j) { return ab[(long)(j - 1) * ld + (kd - 1 + (r - j))]; };
-  int hi = min(n, NBH + kl + CHUNK);
-  for (int pos = 1 + tid; pos <= hi; pos += NT) R[ring_slot(pos)] = b[pos - 1];
-  __syncthreads();
-  int j0 = 1;
-  while (j0 <= n - 1) {
-    if (j0 + NBH - 1 + kl > hi && hi < n) {
-      // rows up to j0+NBH-1+kl; the slots reused belong to rows below j0
-      const int top = min(n, j0 + NBH - 1 + kl + CHUNK);
-      for (int pos = hi + 1 + tid; pos <= top; pos += NT) R[ring_slot(pos)] = b[pos - 1];
-      hi = top;
-      __syncthreads();
+// The columns of AB from j0 on, in step order: entry r of a column lies at
+// p[r - j0].  Moves on to the next column with every step and stays at the
+// last one that is used.
+struct BandCursor {
+  const double* p;
+  int left, step;   // columns to go; the distance of one
+  __device__ __forceinline__ void next() {
+    p += left > 0 ? step : 0;
+    left--;
+  }
+};
+
+// the band entries of the next D steps, for the rows off[e] from the block's first
+template <int E, int D>
+__device__ __forceinline__ void band_load(double (&lt)[E][D], BandCursor& next, const int (&off)[E]) {
+#pragma unroll
+  for (int q = 0; q < D; q++) {
+#pragma unroll
+    for (int e = 0; e < E; e++) lt[e][q] = next.p[off[e]];
+    next.next();
+  }
+}
+
+// the tail's steps of one block, the first D of which have their band entries
+// in lt.  valid(e, sc): the step is taken and the row is within its band (ALL:
+// they all are).
+template <bool ALL, bool BACK, int E, int D, class Valid>
+__device__ __forceinline__ void band_tail(double (&v)[E], double (&lt)[E][D], const double* T, BandCursor& next,
+                                          const int (&off)[E], Valid valid) {
+#pragma unroll
+  for (int k0 = 0; k0 < NBH; k0 += D) {
+#pragma unroll
+    for (int q = 0; q < D; q++) {
+      const int sc = BACK ? NBH - 1 - (k0 + q) : k0 + q;
+      const double ts = T[sc];
+#pragma unroll
+      for (int e = 0; e < E; e++) {
+        const double y = BACK ? v[e] - ts * lt[e][q] : v[e] + lt[e][q] * ts;
+        v[e] = ALL || valid(e, sc) ? y : v[e];
+      }
     }
-    // the block: steps j0 .. j1, the pivots of steps j0+1 .. j1 inside the head
-    const int jp = j0 + lane;
-    const bool out = lane >= 1 && jp <= n - 1 && ipiv[jp - 1] > j0 + NBH - 1;
+    if (k0 + D < NBH) band_load(lt, next, off);
+  }
+}
+
+// forward: L y = P b, in place on b.  (ab has NBH entries of padding: lanes
+// beyond a column's band read past it and drop what they read.)
+template <int E, int D>
+__global__ void __launch_bounds__(SOLVE_MAX_TAIL + 64) k_band_forward(const double* __restrict__ ab,
+                                                                      const int32_t* __restrict__ ipiv, double* b,
+                                                                      int n, int kl, int ku) {
+  __shared__ double R[RING];
+  __shared__ double T[NBH];   // -b(j) of the block's steps
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const long ld = 2 * kl + ku + 1;
+  if (kl == 0 || n < 2) return;
+  int hi = min(n, NBH + kl + CHUNK);
+  for (int pos = 1 + tid; pos <= hi; pos += blockDim.x) R[ring_slot(pos)] = b[pos - 1];
+  __syncthreads();
+  // L(r, j) = AB(kl+ku+1+r-j, j), 1-based; columns past n-1 are not used
+  auto columns = [&](int j0) {
+    const int j = min(j0, n - 1);
+    return BandCursor{ab + ((long)(j - 1) * ld + (kl + ku + j0 - j)), n - 1 - j, (int)ld - 1};
+  };
+  auto pivots = [&](int j0) { return ipiv[min(j0 + lane, n - 1) - 1]; };
+  // the block from j0: steps j0 .. j0+nb-1, the pivots of all but the first inside the head
+  auto steps = [&](int j0, int pl) {
+    const bool out = lane >= 1 && j0 + lane <= n - 1 && pl > j0 + NBH - 1;
     const unsigned long long m = __ballot(out);
-    const int f = m ? __ffsll((long long)m) - 1 : NBH;
-    const int j1 = min(min(j0 + f - 1, j0 + NBH - 1), n - 1);
-    const int nb = j1 - j0 + 1;
-    if (tid == 0) {
-      const int l0 = ipiv[j0 - 1];
-      if (l0 != j0) {
+    return min(min(m ? __ffsll((long long)m) - 1 : NBH, NBH), n - j0);
+  };
+  int pl = pivots(1);
+  if (wave == 0) {
+    double lc[1][NBH];
+    const int off[1] = {lane};
+    BandCursor next = columns(1);
+    band_load(lc, next, off);
+    for (int j0 = 1; j0 <= n - 1;) {
+      const int nb = steps(j0, pl), jn = j0 + nb, pn = pivots(jn);
+      int me = lane;   // not known outside the loop, or 64 comparisons of it would be kept
+      asm volatile("" : "+v"(me));
+      const int l0 = __builtin_amdgcn_readfirstlane(pl);
+      if (l0 != j0 && lane == 0) {
         const double t0 = R[ring_slot(j0)];
         R[ring_slot(j0)] = R[ring_slot(l0)];
         R[ring_slot(l0)] = t0;
       }
-    }
-    {
-      // wave w stages columns w, w+nw, ...: up to 16 loads in flight per lane,
-      // from clamped (valid) band entries, then the masked stores
-      const int nw = NT >> 6, wv = tid >> 6;
-      for (int c0 = 0; c0 < NBH; c0 += 16 * nw) {
-        double tmp[16];
-#pragma unroll
-        for (int q = 0; q < 16; q++) {
-          const int j = min(j0 + min(c0 + q * nw + wv, nb - 1), n - 1);
-          tmp[q] = Lg(min(max(j0 + lane, j + 1), j + kl), j);
-        }
-#pragma unroll
-        for (int q = 0; q < 16; q++) {
-          const int sc = c0 + q * nw + wv, j = j0 + sc, row = j0 + lane;
-          if (sc < NBH) Lh[sc][lane] = (sc < nb && lane > sc && row <= min(n, j + kl)) ? tmp[q] : 0.0;
-        }
-      }
-    }
-    __syncthreads();
-    if (tid < 64) {
-      double v = (j0 + lane <= n) ? R[ring_slot(j0 + lane)] : 0.0;
-      // the block's pivot rows, one per lane, and each step's multiplier kept
-      // in the step's lane: no memory operation inside the step loop
-      const int pl = ipiv[min(j0 + lane, n - 1) - 1];
-      double tv = 0.0;
-      // a full block with no interchange after its first step and a band at
-      // least a head wide (the common case): each step is one lane read and
-      // one masked multiply-add
+      double v = (j0 + lane <= n) ? R[ring_slot(j0 + lane)] : 0.0, tv = 0.0;
       const bool swaps = __ballot(lane >= 1 && lane < nb && pl != j0 + lane) != 0;
-      const bool fast = nb == NBH && !swaps && kl >= NBH && j0 + NBH - 1 <= n;
-      if (fast) {
+      if (nb == NBH && !swaps && kl >= NBH) {
+        // each step is one lane read and one multiply-add; what it leaves in
+        // the lanes of finished rows is not used
 #pragma unroll
-        for (int half = 0; half < 2; half++) {
-          double lc[NBH / 2];
-#pragma unroll
-          for (int q = 0; q < NBH / 2; q++) lc[q] = Lh[half * (NBH / 2) + q][lane];
-#pragma unroll
-          for (int q = 0; q < NBH / 2; q++) {
-            const int sc = half * (NBH / 2) + q;
-            const double temp = -1.0 * readlane_f64(v, sc);
-            if (lane == sc) tv = temp;
-            if (lane > sc) v = v + lc[q] * temp;
-          }
+        for (int sc = 0; sc < NBH; sc++) {
+          const double temp = -1.0 * readlane_f64(v, sc);
+          tv = me == sc ? temp : tv;
+          v = v + lc[0][sc] * temp;
         }
-      }
-      // the steps in two halves, each with its column of the triangle in
-      // registers and constant lane indices
+        v = -1.0 * tv;
+      } else {
 #pragma unroll
-      for (int half = 0; half < 2 && !fast; half++) {
-        double lc[NBH / 2];
-#pragma unroll
-        for (int q = 0; q < NBH / 2; q++) lc[q] = Lh[half * (NBH / 2) + q][lane];
-#pragma unroll
-        for (int q = 0; q < NBH / 2; q++) {
-          const int sc = half * (NBH / 2) + q;
+        for (int sc = 0; sc < NBH; sc++) {
           if (sc < nb) {
             const int j = j0 + sc;
             if (sc > 0) {
               const int l = __builtin_amdgcn_readlane(pl, sc);
               if (l != j) {
                 const double a = readlane_f64(v, sc), c = readlane_f64(v, l - j0);
-                if (lane == sc) v = c;
-                if (lane == l - j0) v = a;
+                if (me == sc) v = c;
+                if (me == l - j0) v = a;
               }
             }
             const double temp = -1.0 * readlane_f64(v, sc);
-            if (lane == sc) tv = temp;
-            if (lane > sc && j0 + lane <= min(n, j + kl)) v = v + lc[q] * temp;
+            tv = me == sc ? temp : tv;
+            const double y = v + lc[0][sc] * temp;
+            v = me > sc && j0 + me <= min(n, j + kl) ? y : v;
           }
         }
       }
       T[lane] = tv;
-      if (lane < nb) b[j0 + lane - 1] = v;                    // y(j0 .. j1): final
+      if (lane < nb) b[j0 + lane - 1] = v;                    // y(j0 .. j0+nb-1): final
       else if (j0 + lane <= n) R[ring_slot(j0 + lane)] = v;   // head rows of the next block
+      __syncthreads();
+      next = columns(jn);   // while the tail works on this block
+      band_load(lc, next, off);
+      __syncthreads();
+      j0 = jn;
+      pl = pn;
     }
-    __syncthreads();
-    // tail rows j0+NBH .. j1+kl
+    if (lane == 0) b[n - 1] = R[ring_slot(n)];
+  } else {
+    const int nt = blockDim.x - 64;
+    int row[E], off[E];   // rows below the head, and within the band of every step
+    bool full = true;
+    double lt[E][D], v[E];
 #pragma unroll
     for (int e = 0; e < E; e++) {
-      const int t = tid + e * NT, r = j0 + NBH + t;
-      const bool act = t < kl && r <= min(n, j1 + kl);
-      double v = act ? R[ring_slot(r)] : 0.0;
-#pragma unroll
-      for (int half = 0; half < 2; half++) {
-        // unconditional loads from clamped (valid) band entries, all in flight at once
-        double lt[NBH / 2];
-#pragma unroll
-        for (int q = 0; q < NBH / 2; q++) {
-          const int j = min(j0 + half * (NBH / 2) + q, j1);
-          lt[q] = Lg(min(max(r, j + 1), j + kl), j);
-        }
-#pragma unroll
-        for (int q = 0; q < NBH / 2; q++) {
-          const int sc = half * (NBH / 2) + q, j = j0 + sc;
-          if (sc < nb && r <= j + kl) v = v + lt[q] * T[sc];
-        }
-      }
-      if (act) R[ring_slot(r)] = v;
+      row[e] = tid - 64 + e * nt;
+      off[e] = NBH + min(row[e], kl - 1);
+      full = full && NBH + 64 * (wave - 1) + 63 + e * nt <= kl;
     }
-    __syncthreads();
-    j0 = j1 + 1;
+    for (int j0 = 1; j0 <= n - 1;) {
+      const int nb = steps(j0, pl), jn = j0 + nb;
+      pl = pivots(jn);
+      BandCursor next = columns(j0);   // while the head works on this block
+      band_load(lt, next, off);
+      // the rows of the next block; the slots reused belong to rows below j0
+      if (const int want = min(n, jn + NBH - 1 + kl); hi < want) {
+        const int top = min(n, want + CHUNK);
+        for (int pos = hi + 1 + tid - 64; pos <= top; pos += nt) R[ring_slot(pos)] = b[pos - 1];
+        hi = top;
+      }
+      __syncthreads();
+#pragma unroll
+      for (int e = 0; e < E; e++) v[e] = R[ring_slot(min(j0 + NBH + row[e], n))];
+      int room[E];   // steps before the row enters the band
+#pragma unroll
+      for (int e = 0; e < E; e++) {
+        room[e] = NBH + row[e] - kl;
+        asm volatile("" : "+v"(room[e]));
+      }
+      auto valid = [&](int e, int sc) { return sc < nb && room[e] <= sc; };
+      if (full && nb == NBH) band_tail<true, false>(v, lt, T, next, off, valid);
+      else band_tail<false, false>(v, lt, T, next, off, valid);
+#pragma unroll
+      for (int e = 0; e < E; e++) {
+        const int r = j0 + NBH + row[e];
+        if (row[e] < kl && r <= min(n, jn - 1 + kl)) R[ring_slot(r)] = v[e];
+      }
+      __syncthreads();
+      j0 = jn;
+    }
   }
-  if (tid == 0) b[n - 1] = R[ring_slot(n)];
 }
 
 // backward: U x = y (DTBSV, upper, non-unit, bandwidth kl+ku), in place on b
-template <int E>   // tail rows per thread
-__global__ void __launch_bounds__(SOLVE_MAX_THREADS) k_band_backward(const double* __restrict__ ab, double* b,
-                                                                     int n, int kl, int ku) {
+template <int E, int D>
+__global__ void __launch_bounds__(SOLVE_MAX_TAIL + 64) k_band_backward(const double* __restrict__ ab, double* b,
+                                                                       int n, int kl, int ku) {
   __shared__ double R[RING];
-  __shared__ double Uh[NBH][NBH];   // Uh[s][r] = U(j0+r, j0+s), r < s
-  __shared__ double X[NBH];         // x(j) of the block's steps
-  __shared__ int F[NBH];            // step taken (b(j) != 0)
-  const int tid = threadIdx.x, NT = blockDim.x, lane = tid & 63;
+  __shared__ double X[NBH];              // x(j) of the block's steps
+  __shared__ unsigned long long taken;   // the steps taken (b(j) != 0)
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const long ld = 2 * kl + ku + 1;
   const int kk = kl + ku;   // U(i, j) = AB(kk+1+i-j, j)
-  auto Ug = [&](int i, int j) { return ab[(long)(j - 1) * ld + (kk + i - j)]; };
   int lo = max(1, n - NBH - kk - CHUNK + 1);
-  for (int pos = lo + tid; pos <= n; pos += NT) R[ring_slot(pos)] = b[pos - 1];
+  for (int pos = lo + tid; pos <= n; pos += blockDim.x) R[ring_slot(pos)] = b[pos - 1];
   __syncthreads();
-  int j1 = n;
-  while (j1 >= 1) {
-    const int j0 = max(1, j1 - NBH + 1), nb = j1 - j0 + 1;
-    if (j0 - kk < lo && lo > 1) {
-      const int bot = max(1, j0 - kk - CHUNK);
-      for (int pos = bot + tid; pos < lo; pos += NT) R[ring_slot(pos)] = b[pos - 1];
-      lo = bot;
-      __syncthreads();
-    }
-    {
-      // as in the forward pass; r == sc is the diagonal U(j,j)
-      const int nw = NT >> 6, wv = tid >> 6;
-      for (int c0 = 0; c0 < NBH; c0 += 16 * nw) {
-        double tmp[16];
+  // from column j0+NBH-1 down (columns past n, in a matrix smaller than a block,
+  // are read from the last one)
+  auto columns = [&](int j0) {
+    const int j = min(j0 + NBH - 1, n);
+    return BandCursor{ab + ((long)(j - 1) * ld + (kk + j0 - j)), j - j0, 1 - (int)ld};
+  };
+  if (wave == 0) {
+    auto diag = [&](int j0) { return ab[(long)(min(j0 + lane, n) - 1) * ld + kk]; };
+    int j1 = n, j0 = max(1, n - NBH + 1);
+    BandCursor next = columns(j0);
+    double uc[1][NBH], dg = diag(j0);   // uc[0][k]: step k, column j0 + NBH-1 - k
+    const int off[1] = {lane};
+    band_load(uc, next, off);
+    while (j1 >= 1) {
+      const int nb = j1 - j0 + 1, jn = max(1, j0 - NBH);
+      int me = lane;
+      asm volatile("" : "+v"(me));
+      double v = (lane < nb) ? R[ring_slot(j0 + lane)] : 0.0, xv = 0.0;
+      unsigned long long tk = 0;
+      // Quotients from the reciprocals of the diagonal, correctly rounded by
+      // two corrections (Markstein) while no exponent is extreme: a chain of 5
+      // operations instead of about 14
+      const double rd = 1.0 / dg, u = dg;
+      const bool mild = fabs(u) > 0x1p-400 && fabs(u) < 0x1p400;
+      if (nb == NBH && kk >= NBH && __ballot(!mild) == 0) {
+        double vb = 0.0;
 #pragma unroll
-        for (int q = 0; q < 16; q++) {
-          const int j = j0 + min(c0 + q * nw + wv, nb - 1);
-          tmp[q] = Ug(max(min(j0 + lane, j), j - kk), j);
+        for (int k = 0; k < NBH; k++) {
+          const int sc = NBH - 1 - k;
+          const double bj = readlane_f64(v, sc), us = readlane_f64(u, sc);
+          const double rs = readlane_f64(rd, sc), q0 = bj * rs, q1 = __fma_rn(__fma_rn(-q0, us, bj), rs, q0);
+          double x = __fma_rn(__fma_rn(-q1, us, bj), rs, q1);
+          const unsigned long long bits = (unsigned long long)__double_as_longlong(bj);
+          const bool take = (bits << 1) != 0;
+          if ((unsigned)((bits >> 52) & 0x7ff) - 523u > 1000u && take) x = bj / us;
+          vb = me == sc ? v : vb;
+          xv = me == sc ? x : xv;
+          if (take) tk |= 1ull << sc;
+          const double y = v - x * uc[0][k];
+          v = take ? y : v;
         }
+        v = (tk >> lane) & 1 ? xv : vb;
+      } else {
+        // the band may not reach every head row
 #pragma unroll
-        for (int q = 0; q < 16; q++) {
-          const int sc = c0 + q * nw + wv, j = j0 + sc, row = j0 + lane;
-          if (sc < NBH) Uh[sc][lane] = (sc < nb && lane <= sc && row >= j - kk) ? tmp[q] : 0.0;
-        }
-      }
-    }
-    __syncthreads();
-    if (tid < 64) {
-      double v = (lane < nb) ? R[ring_slot(j0 + lane)] : 0.0;
-      double xv = 0.0;   // x(j) and whether step j was taken, in the step's lane
-      int fv = 0;
-      // the band reaches every head row when kl+ku >= NBH
-      const bool wide = kk >= NBH;
-#pragma unroll
-      for (int half = 1; half >= 0; half--) {
-        double uc[NBH / 2];
-#pragma unroll
-        for (int q = 0; q < NBH / 2; q++) uc[q] = Uh[half * (NBH / 2) + q][lane];
-#pragma unroll
-        for (int q = NBH / 2 - 1; q >= 0; q--) {
-          const int sc = half * (NBH / 2) + q;
-          if (sc < nb) {
-            const int j = j0 + sc;
-            const double bj = readlane_f64(v, sc);
-            if (bj != 0.0) {
-              const double x = bj / readlane_f64(uc[q], sc);   // U(j,j)
-              if (lane == sc) v = x;
-              if (lane < sc && (wide || j0 + lane >= j - kk)) v = v - x * uc[q];
-              if (lane == sc) { xv = x; fv = 1; }
-            }
+        for (int k = 0; k < NBH; k++) {
+          const int sc = NBH - 1 - k;
+          const double bj = readlane_f64(v, sc);
+          if (sc < nb && bj != 0.0) {
+            const double x = bj / readlane_f64(u, sc);
+            if (me == sc) v = xv = x;
+            const double y = v - x * uc[0][k];
+            v = me < sc && sc - me <= kk ? y : v;
+            tk |= 1ull << sc;
           }
         }
       }
       X[lane] = xv;
-      F[lane] = fv;
+      if (lane == 0) taken = tk;
       if (lane < nb) b[j0 + lane - 1] = v;   // x(j0 .. j1): final
+      __syncthreads();
+      dg = diag(jn);   // while the tail works on this block
+      next = columns(jn);
+      band_load(uc, next, off);
+      __syncthreads();
+      j1 = j0 - 1;
+      j0 = jn;
     }
-    __syncthreads();
-    // tail rows j0-1 down to j0-kk
+  } else {
+    const int nt = blockDim.x - 64;
+    int row[E], off[E];   // rows above the head: j0-1-row, and within the band of every step
+    bool full = true;
+    double lt[E][D], v[E];
+    int j1 = n, j0 = max(1, n - NBH + 1);
 #pragma unroll
     for (int e = 0; e < E; e++) {
-      const int t = tid + e * NT, i = j0 - 1 - t;
-      const bool act = t < kk && i >= 1;
-      double v = act ? R[ring_slot(i)] : 0.0;
-#pragma unroll
-      for (int half = 1; half >= 0; half--) {
-        double ut[NBH / 2];
-#pragma unroll
-        for (int q = 0; q < NBH / 2; q++) {
-          const int j = min(j0 + half * (NBH / 2) + q, j1);
-          ut[q] = Ug(min(max(i, j - kk), j - 1 < 1 ? j : j - 1), j);
-        }
-#pragma unroll
-        for (int q = NBH / 2 - 1; q >= 0; q--) {
-          const int sc = half * (NBH / 2) + q, j = j0 + sc;
-          if (sc < nb && F[sc] && i >= j - kk) v = v - X[sc] * ut[q];
-        }
-      }
-      if (act) R[ring_slot(i)] = v;
+      row[e] = tid - 64 + e * nt;
+      off[e] = -1 - min(row[e], kk - 1);
+      full = full && 64 * (wave - 1) + 63 + e * nt <= kk - NBH;
     }
-    __syncthreads();
-    j1 = j0 - 1;
+    while (j1 >= 1) {
+      const int jn = max(1, j0 - NBH);
+      BandCursor next = columns(j0);   // while the head works on this block
+      band_load(lt, next, off);
+      // the rows of the next block; the slots reused belong to rows above j1
+      if (const int want = max(1, jn - kk); lo > want) {
+        const int bot = max(1, want - CHUNK);
+        for (int pos = bot + tid - 64; pos < lo; pos += nt) R[ring_slot(pos)] = b[pos - 1];
+        lo = bot;
+      }
+      __syncthreads();
+      const unsigned long long tk = taken;
+      const bool every = __builtin_amdgcn_readfirstlane((int)(tk & (tk >> 32))) == -1;
+#pragma unroll
+      for (int e = 0; e < E; e++) v[e] = R[ring_slot(max(j0 - 1 - row[e], 1))];
+      int room[E];   // steps from which on the row is in the band
+#pragma unroll
+      for (int e = 0; e < E; e++) {
+        room[e] = kk - 1 - row[e];
+        asm volatile("" : "+v"(room[e]));
+      }
+      auto valid = [&](int e, int sc) { return ((tk >> sc) & 1) && sc <= room[e]; };
+      if (full && every) band_tail<true, true>(v, lt, X, next, off, valid);
+      else band_tail<false, true>(v, lt, X, next, off, valid);
+#pragma unroll
+      for (int e = 0; e < E; e++)
+        if (row[e] < kk && j0 - 1 - row[e] >= 1) R[ring_slot(j0 - 1 - row[e])] = v[e];
+      __syncthreads();
+      j1 = j0 - 1;
+      j0 = jn;
+    }
   }
 }
 
@@ -743,7 +809,7 @@ int direct_alloc(Context& c) {
     return PT_ERR_UNSUPPORTED;
   }
   const size_t ld = (size_t)(2 * t.dkl + t.dku + 1);
-  if (hipMalloc((void**)&c.dAB, sizeof(double) * ld * (size_t)t.dn) != hipSuccess ||
+  if (hipMalloc((void**)&c.dAB, sizeof(double) * (ld * (size_t)t.dn + NBH)) != hipSuccess ||
       hipMalloc((void**)&c.dRow, sizeof(double) * (size_t)t.dn) != hipSuccess ||
       hipMalloc((void**)&c.dB, sizeof(double) * (size_t)t.dn) != hipSuccess ||
       hipMalloc((void**)&c.dipiv, sizeof(int32_t) * (size_t)t.dn) != hipSuccess ||
@@ -832,31 +898,33 @@ int solve_sf_equation(Context& c) {
   const SfArgs a = sf_args(c);
   hipLaunchKernelGGL(k_sf_buoyancy, dim3((t.dn + 255) / 256), dim3(256), 0, c.stream, a, c.Tbuoy, c.Cbuoy, c.dRow,
                      c.P.RaT, c.P.RaC, c.dB);
-  // one workgroup per triangular solve, sized to its band: 64-thread waves,
-  // at most 1024 threads, E band rows per thread
-  auto shape = [](int band, int& nt, int& e) {
-    nt = std::min(SOLVE_MAX_THREADS, ((band + 63) / 64) * 64);
-    e = (band + nt - 1) / nt;
+  // one workgroup per triangular solve: the head's wavefront, and tail
+  // wavefronts with E rows per thread that load D steps at a time, as the
+  // band's height needs and the registers allow.  (E, D) = (2, 32) against
+  // (2, 16) with up to 15 tail wavefronts, 20x210 (bands 633 and 1266): 1.46
+  // and 1.65 ms; (4, 8) against (4, 16), which spills, 20x250 (753 and 1506):
+  // 3.2 and 6.4 ms; 4.6 ms before.
+  auto run = [&](int band, auto launch) {
+    if (band <= SOLVE_MAX_TAIL) launch(std::integral_constant<int, 1>{}, std::integral_constant<int, 64>{}, band);
+    else if (band <= 2 * SOLVE_MAX_TAIL)
+      launch(std::integral_constant<int, 2>{}, std::integral_constant<int, 32>{}, band);
+    else launch(std::integral_constant<int, 4>{}, std::integral_constant<int, 8>{}, band);
   };
-  int ntf, ef, ntb, eb;
-  shape(t.dkl, ntf, ef);
-  shape(t.dkl + t.dku, ntb, eb);
-  if (ef > 4 || eb > 4) {
+  auto threads = [](int band, int e) { return 64 + (((band + e - 1) / e + 63) & ~63); };
+  if (t.dkl + t.dku > 4 * SOLVE_MAX_TAIL) {
     set_error("direct solver: band too wide for the solve kernels");
     return PT_ERR_UNSUPPORTED;
   }
-  auto fwd = [&](auto kern) {
-    hipLaunchKernelGGL(kern, dim3(1), dim3(ntf), 0, c.stream, c.dAB, c.dipiv, c.dB, t.dn, t.dkl, t.dku);
-  };
-  auto bwd = [&](auto kern) {
-    hipLaunchKernelGGL(kern, dim3(1), dim3(ntb), 0, c.stream, c.dAB, c.dB, t.dn, t.dkl, t.dku);
-  };
-  if (ef == 1) fwd(k_band_forward<1>);
-  else if (ef == 2) fwd(k_band_forward<2>);
-  else fwd(k_band_forward<4>);
-  if (eb == 1) bwd(k_band_backward<1>);
-  else if (eb == 2) bwd(k_band_backward<2>);
-  else bwd(k_band_backward<4>);
+  run(t.dkl, [&](auto e, auto d, int band) {
+    constexpr int E = decltype(e)::value, D = decltype(d)::value;
+    hipLaunchKernelGGL((k_band_forward<E, D>), dim3(1), dim3(threads(band, E)), 0, c.stream, c.dAB, c.dipiv, c.dB,
+                       t.dn, t.dkl, t.dku);
+  });
+  run(t.dkl + t.dku, [&](auto e, auto d, int band) {
+    constexpr int E = decltype(e)::value, D = decltype(d)::value;
+    hipLaunchKernelGGL((k_band_backward<E, D>), dim3(1), dim3(threads(band, E)), 0, c.stream, c.dAB, c.dB, t.dn,
+                       t.dkl, t.dku);
+  });
   dim3 b16(64, 4), g((t.nx + 7 + 63) / 64, (t.nz + 7 + 3) / 4);
   hipLaunchKernelGGL(k_sf_scatter, g, b16, 0, c.stream, a, c.dB, c.SF);
   c.solves++;
