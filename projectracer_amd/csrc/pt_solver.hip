@@ -921,6 +921,25 @@ __global__ void k_vis_bcs_tb(double* v, int n, int m, int p) {
   v[IDX(i, m + k, p)] = v[IDX(i, m - k, p)];
 }
 
+// v(i,k) = x with its images (n, m >= 3): side images, top and bottom images,
+// and the corners' side images of the ghost rows, which hold ghost(k') from
+// before
+template <class Ghost>
+__device__ __forceinline__ void vis_store(double* v, int i, int k, int n, int m, int p, double x, Ghost ghost) {
+  const bool left = i >= 1 && i <= 3, right = i <= n - 1 && i >= n - 3;
+  auto image = [&](int kg) {
+    const double old = ghost(kg);
+    v[IDX(i, kg, p)] = x;
+    if (left) v[IDX(-i, kg, p)] = old;
+    if (right) v[IDX(2 * n - i, kg, p)] = old;
+  };
+  v[IDX(i, k, p)] = x;
+  if (left) v[IDX(-i, k, p)] = x;
+  if (right) v[IDX(2 * n - i, k, p)] = x;
+  if (k >= 1 && k <= 3) image(-k);
+  if (k <= m - 1 && k >= m - 3) image(2 * m - k);
+}
+
 // viscosityBCs_initialize (PS/iterative_solver.f90:636-664)
 __global__ void k_vis_bcs_init_boundary(double* v, const double* f, int n, int m, int p, int fn, int fm, int fp) {
   int t = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1033,11 +1052,73 @@ __global__ void k_test_eig(VisSet s, double* ratio, double* dts, int n, int m, i
   if (tid == 0) partial[blockIdx.y * gridDim.x + blockIdx.x] = red[0];
 }
 
+// one update from the gradients' vsmooth, and viscosityBCs.  A thread writes
+// its node's images too; those in the corners (side images of the ghost rows)
+// take the ghost rows as they were before, as the side pass does.
 __global__ void k_vis_update(double* v, const double* sm, int n, int m, int p, double c) {
   int i = blockIdx.x * blockDim.x + threadIdx.x, k = blockIdx.y * blockDim.y + threadIdx.y;
   if (i > n || k > m) return;
   long g = IDX(i, k, p);
-  v[g] = v[g] + c * sm[g];
+  vis_store(v, i, k, n, m, p, v[g] + c * sm[g], [&](int kg) { return v[IDX(i, kg, p)]; });
+}
+
+// Several updates per launch, for the iterations between which nothing is
+// asked of the gradients: v = v + cc dtv (vxx + vzz), each with viscosityBCs.
+// A workgroup holds its tile and as many rows and columns around it as there
+// are updates in LDS, in two copies; what its edge lacks spoils one more row
+// per update and stops short of the tile.  Neighbours across the domain's edge
+// are the mirrored ones.  Bound by launches: an update took four (gradients,
+// update, two of ghosts), 3.8 + 2.5 + 2.3 + 2.4 us on average over the levels
+// of 1024x256, and 3 to 6 of them in one launch take 9.0.
+constexpr int VIS_ITS = 6;             // updates per launch at most
+constexpr int VIS_TZ = 16;             // tile rows; a tile is 64 - 2 its columns wide
+constexpr int VIS_ROWS = VIS_TZ + 2 * VIS_ITS;
+struct VisSmooth {
+  const double* in;
+  double* out;
+  double cc[VIS_ITS];
+  double dr2, ds2, rdr2, rds2, dtv;
+  int n, m, p, its, ghosts;   // ghosts: the last launch, which leaves them
+};
+
+template <bool PW2>
+__global__ void __launch_bounds__(256) k_vis_smooth(VisSmooth a) {
+  __shared__ double V[2][VIS_ROWS][64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int H = a.its, n = a.n, m = a.m, p = a.p;
+  const int x0 = blockIdx.x * (64 - 2 * H) - H, z0 = blockIdx.y * VIS_TZ - H;   // the tile's corner with its surroundings
+  const int rows = VIS_TZ + 2 * H, i = x0 + lane;
+  const int il = max(i == 0 ? lane + 1 : lane - 1, 0), ir = min(i == n ? lane - 1 : lane + 1, 63);
+  for (int r = wave; r < rows; r += 4)
+    V[0][r][lane] = a.in[IDX(min(max(i, 0), n), min(max(z0 + r, 0), m), p)];
+  __syncthreads();
+  for (int it = 0; it < H; it++) {
+    const double(*A)[64] = V[it & 1];
+    double(*B)[64] = V[(it + 1) & 1];
+    for (int r = wave; r < rows; r += 4) {
+      const int k = z0 + r, rd = max(k == 0 ? r + 1 : r - 1, 0), ru = min(k == m ? r - 1 : r + 1, rows - 1);
+      const double v = A[r][lane];
+      double sxx = 0.0, szz = 0.0;
+      sxx = sxx + A[r][il];
+      sxx = sxx + (-2.0) * v;
+      sxx = sxx + A[r][ir];
+      szz = szz + A[rd][lane];
+      szz = szz + (-2.0) * v;
+      szz = szz + A[ru][lane];
+      const double xp = quot<PW2>(sxx, a.dr2, a.rdr2) + quot<PW2>(szz, a.ds2, a.rds2);
+      B[r][lane] = v + a.cc[it] * (a.dtv * xp);
+    }
+    __syncthreads();
+  }
+  if (lane < H || lane >= 64 - H || i > n) return;
+  for (int r = H + wave; r < H + VIS_TZ; r += 4) {
+    const int k = z0 + r;
+    if (k > m) break;
+    if (a.ghosts)
+      vis_store(a.out, i, k, n, m, p, V[H & 1][r][lane], [&](int) { return V[(H + 1) & 1][r][lane]; });
+    else
+      a.out[IDX(i, k, p)] = V[H & 1][r][lane];
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -1540,7 +1621,6 @@ static int smoother_vis(Context& c, int l, VisSet& vs, int interpolate) {
     int cols = (g.n + 1) * 3;
     hipLaunchKernelGGL(k_vis_bcs_tb, dim3((cols + 255) / 256), dim3(256), 0, c.stream, vs.vis, g.n, g.m, g.pitch);
   };
-  bcs();
   int option, Niter;
   double lb, la;
   if (interpolate == 0) { option = 1; Niter = 3; lb = -3.0; la = -2.0; }
@@ -1562,6 +1642,35 @@ static int smoother_vis(Context& c, int l, VisSet& vs, int interpolate) {
     // k_test_eig's RKC1 form with unit ellipse axes (eR/1 and eI/1 are exact)
     ae = 1.0; be = 1.0;
     ctemp = -(c.P.courant_stream * 2.0);
+  }
+  auto factor = [&](int nn) {
+    const int ntemp = Niter - nn + 1;
+    const double cc = 2.0 / (-lb - la + (lb - la) * std::cos((double)(2 * ntemp - 1) * 3.1415926535897932 / (double)(2 * Niter)));
+    return 0.99 * cc;
+  };
+  // the first pass asks nothing of the gradients: its updates go several to a
+  // launch, from vis to vsmooth (scratch until the gradients are taken) and
+  // back.  (A grid less than 3 wide mirrors ghosts of ghosts.)
+  if (!ivis0 && Niter >= 2 && g.n >= 3 && g.m >= 3) {
+    VisSmooth a;
+    a.dr2 = g.dr2; a.ds2 = g.ds2; a.rdr2 = 1.0 / g.dr2; a.rds2 = 1.0 / g.ds2; a.dtv = t.dt_vis[l];
+    a.n = g.n; a.m = g.m; a.p = g.pitch;
+    const int launches = 2 * ((Niter + 2 * VIS_ITS - 1) / (2 * VIS_ITS));
+    for (int k = 0, nn = 1; k < launches; k++, nn += a.its) {
+      a.its = (Niter - nn + 1 + launches - k - 1) / (launches - k);
+      for (int q = 0; q < a.its; q++) a.cc[q] = factor(nn + q);
+      a.in = k & 1 ? vs.vsmooth : vs.vis;
+      a.out = k & 1 ? vs.vis : vs.vsmooth;
+      a.ghosts = k + 1 == launches;
+      const dim3 grid((g.n + 64 - 2 * a.its) / (64 - 2 * a.its), (g.m + VIS_TZ) / VIS_TZ);
+      if (pow2(g.dr2) && pow2(g.ds2)) hipLaunchKernelGGL(k_vis_smooth<true>, grid, dim3(256), 0, c.stream, a);
+      else hipLaunchKernelGGL(k_vis_smooth<false>, grid, dim3(256), 0, c.stream, a);
+    }
+    Nvis_store++;
+    if (option == 1) { Niter = 6; lb = -2.0; la = -1.0; }
+    n++;
+  } else {
+    bcs();
   }
   for (;;) {
     for (int nn = nn_store; nn <= Niter; nn++) {
@@ -1590,11 +1699,8 @@ static int smoother_vis(Context& c, int l, VisSet& vs, int interpolate) {
         trigger = true;
         break;
       }
-      int ntemp = Niter - nn + 1;
-      double cc = 2.0 / (-lb - la + (lb - la) * std::cos((double)(2 * ntemp - 1) * 3.1415926535897932 / (double)(2 * Niter)));
-      cc = 0.99 * cc;
-      hipLaunchKernelGGL(k_vis_update, gnodes, b16, 0, c.stream, vs.vis, vs.vsmooth, g.n, g.m, g.pitch, cc);
-      bcs();
+      hipLaunchKernelGGL(k_vis_update, gnodes, b16, 0, c.stream, vs.vis, vs.vsmooth, g.n, g.m, g.pitch, factor(nn));
+      if (g.n < 3 || g.m < 3) bcs();
     }
     if (trigger) break;
     Nvis_store++;
