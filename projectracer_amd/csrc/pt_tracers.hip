@@ -761,13 +761,12 @@ __device__ __forceinline__ double filter_nodes(const FilterArgs& a, const Filter
 template <bool COMP, bool PW2>
 __global__ void __launch_bounds__(FILTER_THREADS) k_filter_passes(FilterArgs a, FilterLaunch f) {
   extern __shared__ double fsm[];
-  __shared__ int s_ok[FILTER_KMAX], s_inf;
+  __shared__ int s_ok[FILTER_KMAX], s_bad[FILTER_THREADS / 64];
   constexpr int RB = FILTER_RB;
   const int nx = a.nx, nz = a.nz, K = a.K, tid = threadIdx.x, nthr = blockDim.x;
   const int lane = tid & 63, wave = tid >> 6, nwave = nthr >> 6;
   const int W = a.pitch, ne = a.pitch * a.rows;
   double* const dmax = fsm + 2 * ne;   // [K][nthr]: every thread's part of each check
-  if (tid == 0) s_inf = 0;
   // XCD-aware tiles: workgroups are dealt round-robin over the 8 XCDs; each
   // XCD gets one contiguous band of tiles, the same in every launch, so that
   // most of what a tile reads is in its own L2
@@ -785,9 +784,11 @@ __global__ void __launch_bounds__(FILTER_THREADS) k_filter_passes(FilterArgs a, 
   const int zlo = max(0, cz0 - 2 * K), nrow = min(nz, cz1 - 1 + 2 * K) - zlo + 1;
   // window: element e = row * ncol + column, threads nthr apart
   const int er0 = tid / ncol, ec0 = tid - er0 * ncol, dr = nthr / ncol, dc = nthr - dr * ncol;
+  // (each wavefront leaves what it found in a word of its own, written at
+  // every load, so the flags need no initial value; read after the barrier)
+  bool bad = false;
   auto load = [&](const double* src) {
     int er = er0, ec = ec0;
-    bool bad = false;
     while (er < nrow) {
       constexpr int FB = 5;
       double v[FB];
@@ -808,7 +809,8 @@ __global__ void __launch_bounds__(FILTER_THREADS) k_filter_passes(FilterArgs a, 
           bad |= !(fabs(v[u]) < INFINITY);
         }
     }
-    if (bad) s_inf = 1;
+    const bool any = __ballot(bad) != 0;
+    if (lane == 0) s_bad[wave] = any;
   };
   // the control word, the previous launch's checks (wavefront t takes check
   // t) and the window are loaded together, before the decision
@@ -950,7 +952,7 @@ __global__ void __launch_bounds__(FILTER_THREADS) k_filter_passes(FilterArgs a, 
       __syncthreads();
     }
   }
-  const bool finite = s_inf == 0;
+  const bool finite = __ballot(lane < nwave && s_bad[lane < nwave ? lane : 0] != 0) == 0;
   int at0 = 0;
   double yv[RB];
 #pragma unroll

@@ -1,0 +1,42 @@
+"""The filter loops on fields that are not finite against the loop with a host
+round trip per check (PT_FILTER_HOST=1): an infinity or a NaN in the
+temperature or the composition of one tracer, on a grid with one tile per row
+and on one with several.  Every tile has to see each such value of its window:
+a NaN composition must not be clamped into [0, 1] and an infinite temperature
+must become the NaN that the reference's form makes of it
+(PS/smoother.f90:141-176).  Same arithmetic on both sides: equal pass counts
+and equal fields, NaN for NaN."""
+import numpy as np
+import pytest
+
+from projectracer_amd import Simulation, cases
+
+pytestmark = pytest.mark.gpu
+
+
+def _run(case, monkeypatch, host):
+    monkeypatch.setenv("PT_FILTER_HOST", "1" if host else "0")
+    sim = Simulation(case.params)
+    sim.load_state(case)
+    sim.tracers_to_corners()
+    inf = sim.info()
+    out = (inf["n_comp"], inf["n_temp"]), sim.field("TVIS").copy(), sim.field("CVIS").copy()
+    sim.close()
+    return out
+
+
+@pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan])
+@pytest.mark.parametrize("array", ["Ttr", "Ctr"])
+@pytest.mark.parametrize("nx,nz", [(64, 32), (384, 128)])
+def test_filters_with_a_value_that_is_not_finite(nx, nz, array, value, monkeypatch):
+    print(f"[filters] {nx}x{nz} {array} with {value}", flush=True)
+    case = cases.thermochem(nx=nx, nz=nz, tpc=6, aspect=nx / nz, visT=30.0, visC=0.5, delta_visT=1.2, delta_visC=1.2,
+                            grids=4, mingrid=2)
+    tracers = getattr(case, array)
+    tracers[tracers.size // 2 + 5] = value   # inside a tile, not at its edge
+    tracers[tracers.size // 3] = value
+    device, host = _run(case, monkeypatch, False), _run(case, monkeypatch, True)
+    print(device[0], host[0], int(np.isnan(host[1]).sum()), int(np.isnan(host[2]).sum()), flush=True)
+    assert not np.isfinite(host[1]).all() or not np.isfinite(host[2]).all()
+    assert device[0] == host[0]
+    assert np.array_equal(device[1], host[1], equal_nan=True) and np.array_equal(device[2], host[2], equal_nan=True)
