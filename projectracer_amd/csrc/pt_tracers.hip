@@ -628,6 +628,8 @@ struct FilterArgs {
   int nx, nz, h, p;
   double dr2, ds2, rdr2, rds2;
   double d2[3];         // D2 at offsets 0, 1, 2
+  double dr, ds, d1[5]; // for the general form of a pass
+  double limit;         // values below it stay finite through a launch's passes
   // T: enforceBCs with the isothermal / insulating walls
   int Tbot;
   double Tb, Tt, two_over_d20, H, Htype;
@@ -674,9 +676,10 @@ struct FilterThread {
   bool lowz, highz;     // the window holds rows that read them
 };
 
-// one pass (and the check before it) at a thread's nodes.  FINITE: every value
-// of the window is finite; otherwise the stretched-grid form's Txx = Trr - Tx*0
-// makes a pass NaN where a value it reads is not.
+// one pass (and the check before it) at a thread's nodes.  FINITE: nothing that
+// the launch forms from the window is an infinity or NaN; otherwise the
+// stretched-grid form's Txx = Trr - Tx*0 decides what becomes of them, so it is
+// evaluated as written.
 template <bool COMP, bool PW2, bool FINITE>
 __device__ __forceinline__ double filter_nodes(const FilterArgs& a, const FilterThread& th, const double* X, double* Y,
                                                int k0, double cdts, double* yv) {
@@ -706,10 +709,23 @@ __device__ __forceinline__ double filter_nodes(const FilterArgs& a, const Filter
     sss = sss + a.d2[0] * v;
     sss = sss + a.d2[1] * col[r + 3];
     sss = sss + a.d2[2] * col[r + 4];
-    double Txx = quot<PW2>(srr, a.dr2, a.rdr2), Tzz = quot<PW2>(sss, a.ds2, a.rds2);
-    if constexpr (!FINITE) {
-      Txx = Txx - Txx * 0.0;
-      Tzz = Tzz - Tzz * 0.0;
+    double Txx, Tzz;
+    if constexpr (FINITE) {
+      Txx = quot<PW2>(srr, a.dr2, a.rdr2);
+      Tzz = quot<PW2>(sss, a.ds2, a.rds2);
+    } else {
+      double sr = a.d1[0] * e0;
+      sr = sr + a.d1[1] * e1;
+      sr = sr + a.d1[2] * v;
+      sr = sr + a.d1[3] * e3;
+      sr = sr + a.d1[4] * e4;
+      double ss = a.d1[0] * col[r];
+      ss = ss + a.d1[1] * col[r + 1];
+      ss = ss + a.d1[2] * v;
+      ss = ss + a.d1[3] * col[r + 3];
+      ss = ss + a.d1[4] * col[r + 4];
+      Txx = srr / a.dr2 - sr / a.dr * 0.0;
+      Tzz = sss / a.ds2 - ss / a.ds * 0.0;
     }
     double y = v + cdts * (Txx + Tzz);
     const int k = k0 + r;
@@ -784,8 +800,6 @@ __global__ void __launch_bounds__(FILTER_THREADS) k_filter_passes(FilterArgs a, 
   const int zlo = max(0, cz0 - 2 * K), nrow = min(nz, cz1 - 1 + 2 * K) - zlo + 1;
   // window: element e = row * ncol + column, threads nthr apart
   const int er0 = tid / ncol, ec0 = tid - er0 * ncol, dr = nthr / ncol, dc = nthr - dr * ncol;
-  // (each wavefront leaves what it found in a word of its own, written at
-  // every load, so the flags need no initial value; read after the barrier)
   bool bad = false;
   auto load = [&](const double* src) {
     int er = er0, ec = ec0;
@@ -806,9 +820,13 @@ __global__ void __launch_bounds__(FILTER_THREADS) k_filter_passes(FilterArgs a, 
       for (int u = 0; u < FB; u++)
         if (at[u] >= 0) {
           fsm[at[u]] = v[u];
-          bad |= !(fabs(v[u]) < INFINITY);
+          bad |= !(fabs(v[u]) < a.limit);
         }
     }
+  };
+  // each wavefront leaves what it found in a word of its own, so the flags need
+  // no initial value; read after the barrier that follows
+  auto report = [&]() {
     const bool any = __ballot(bad) != 0;
     if (lane == 0) s_bad[wave] = any;
   };
@@ -932,7 +950,9 @@ __global__ void __launch_bounds__(FILTER_THREADS) k_filter_passes(FilterArgs a, 
     th.At = 2.0 * a.Tt + a.two_over_d20 * (a.Htype * ct + a.H * (1.0 - (0.0 + ct))) * a.ds2;
     th.lowz = a.Tbot == 0 && zlo == 0;
     th.highz = zlo + nrow > nz;
+    bad |= !(fabs(th.Ab) < a.limit && fabs(th.At) < a.limit);
   }
+  report();
   __syncthreads();
   int np = f.k;           // passes this launch makes
   bool final = false;
@@ -949,6 +969,7 @@ __global__ void __launch_bounds__(FILTER_THREADS) k_filter_passes(FilterArgs a, 
       }
       if (t == 0 || edge) return;
       load(f.prev);
+      report();
       __syncthreads();
     }
   }
@@ -1079,10 +1100,21 @@ static FilterPlan filter_plan(int nx, int nz, bool comp) {
   return best;
 }
 
+static double cdts_comp(const Context& c, int j);
+static double cdts_temp(const Context& c, int j);
 static FilterArgs filter_args(const Context& c, bool comp) {
   FilterArgs a = filter_shape(c.T.nx, c.T.nz, comp, c.filter[comp]);
   a.dr2 = c.T.dr2; a.ds2 = c.T.ds2; a.rdr2 = 1.0 / c.T.dr2; a.rds2 = 1.0 / c.T.ds2;
   for (int q = 0; q < 3; q++) a.d2[q] = c.T.D2[3 + q];
+  a.dr = c.T.dr; a.ds = c.T.ds;
+  for (int q = 0; q < 5; q++) a.d1[q] = c.T.D1[q + 1];
+  // a derivative is at most `quotient` times the values it is formed from (the
+  // weights of D1 and D2 sum to 1.5 and 16/3), a pass's result at most `growth`
+  // times them and the ghost rows' constants
+  double step = 0.0;
+  for (int j = 1; j <= 11; j++) step = std::max(step, std::fabs((comp ? cdts_comp : cdts_temp)(c, j)));
+  const double quotient = 6.0 * std::max({1.0, a.rdr2, a.rds2}), growth = 2.0 * (1.0 + 2.0 * step * quotient);
+  a.limit = 0x1p1000 / quotient / std::pow(growth, FILTER_KMAX);
   a.Tbot = c.P.Tbot; a.Tb = c.Tbot_iso; a.Tt = c.Ttop_iso; a.two_over_d20 = 2.0 / c.T.D2[3];
   a.H = c.P.H; a.Htype = c.P.Htype; a.Cvis = c.Cvis;
   a.delta = comp ? c.T.delta_C : c.T.delta_T;

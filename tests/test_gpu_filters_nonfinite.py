@@ -40,3 +40,20 @@ def test_filters_with_a_value_that_is_not_finite(nx, nz, array, value, monkeypat
     assert not np.isfinite(host[1]).all() or not np.isfinite(host[2]).all()
     assert device[0] == host[0]
     assert np.array_equal(device[1], host[1], equal_nan=True) and np.array_equal(device[2], host[2], equal_nan=True)
+
+
+@pytest.mark.parametrize("array,big", [("Ttr", 1.5e308), ("Ctr", 1e300), ("Ctr", 1.5e308)])
+@pytest.mark.parametrize("nx,nz", [(64, 32), (80, 48), (384, 128)])
+def test_filters_with_values_that_overflow(nx, nz, array, big, monkeypatch):
+    """Finite values whose derivatives overflow: the first pass leaves
+    infinities, and the passes after it NaN around them."""
+    print(f"[filters] {nx}x{nz} {array} with {big}", flush=True)
+    case = cases.thermochem(nx=nx, nz=nz, tpc=6, aspect=nx / nz, visT=30.0, visC=0.5, delta_visT=1.2, delta_visC=1.2,
+                            grids=4, mingrid=2)
+    tracers = getattr(case, array)
+    tracers[tracers.size // 2 + 5] = big
+    tracers[tracers.size // 3:tracers.size // 3 + 40] = -big
+    device, host = _run(case, monkeypatch, False), _run(case, monkeypatch, True)
+    print(device[0], host[0], int(np.isnan(host[1]).sum()), int(np.isnan(host[2]).sum()), flush=True)
+    assert device[0] == host[0]
+    assert np.array_equal(device[1], host[1], equal_nan=True) and np.array_equal(device[2], host[2], equal_nan=True)
