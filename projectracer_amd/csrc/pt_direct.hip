@@ -626,15 +626,13 @@ __global__ void __launch_bounds__(SOLVE_MAX_TAIL + 64) k_band_backward(const dou
   int lo = max(1, n - NBH - kk - CHUNK + 1);
   for (int pos = lo + tid; pos <= n; pos += blockDim.x) R[ring_slot(pos)] = b[pos - 1];
   __syncthreads();
-  // from column j0+NBH-1 down (columns past n, in a matrix smaller than a block,
-  // are read from the last one)
+  // from column j0+NBH-1 down (there is one: n >= NBH)
   auto columns = [&](int j0) {
-    const int j = min(j0 + NBH - 1, n);
-    return BandCursor{ab + ((long)(j - 1) * ld + (kk + j0 - j)), j - j0, 1 - (int)ld};
+    return BandCursor{ab + ((long)(j0 + NBH - 2) * ld + (kk + 1 - NBH)), NBH - 1, 1 - (int)ld};
   };
   if (wave == 0) {
-    auto diag = [&](int j0) { return ab[(long)(min(j0 + lane, n) - 1) * ld + kk]; };
-    int j1 = n, j0 = max(1, n - NBH + 1);
+    auto diag = [&](int j0) { return ab[(long)(j0 + lane - 1) * ld + kk]; };
+    int j1 = n, j0 = n - NBH + 1;
     BandCursor next = columns(j0);
     double uc[1][NBH], dg = diag(j0);   // uc[0][k]: step k, column j0 + NBH-1 - k
     const int off[1] = {lane};
@@ -699,7 +697,7 @@ __global__ void __launch_bounds__(SOLVE_MAX_TAIL + 64) k_band_backward(const dou
     int row[E], off[E];   // rows above the head: j0-1-row, and within the band of every step
     bool full = true;
     double lt[E][D], v[E];
-    int j1 = n, j0 = max(1, n - NBH + 1);
+    int j1 = n, j0 = n - NBH + 1;
 #pragma unroll
     for (int e = 0; e < E; e++) {
       row[e] = tid - 64 + e * nt;
@@ -806,6 +804,10 @@ int direct_alloc(Context& c) {
   if (t.dkl + t.dku + NBH + CHUNK >= RING) {   // the solves' LDS window
     set_error("direct solver: band width " + std::to_string(t.dkl + t.dku) + " exceeds " +
               std::to_string(RING - NBH - CHUNK - 1));
+    return PT_ERR_UNSUPPORTED;
+  }
+  if (t.dn < NBH) {   // the backward solve's blocks are whole ones
+    set_error("direct solver: fewer than " + std::to_string(NBH) + " unknowns");
     return PT_ERR_UNSUPPORTED;
   }
   const size_t ld = (size_t)(2 * t.dkl + t.dku + 1);
