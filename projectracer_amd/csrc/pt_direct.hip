@@ -854,10 +854,8 @@ int build_sf_matrix(Context& c) {
   const int rows = t.dkl + LU_NB, kv = t.dkl + t.dku;
   auto factor = [&](auto qc) -> int {
     constexpr int Q = decltype(qc)::value;
-    // set once per process (a thread-safe static initialisation)
-    static const hipError_t attr_rc = hipFuncSetAttribute(
-        (const void*)k_lu_trailing<Q>, hipFuncAttributeMaxDynamicSharedMemorySize, LU_LDS_LIMIT);
-    PT_HIP(attr_rc);
+    static OncePerDevice lds;
+    PT_TRY(allow_lds(c, lds, k_lu_trailing<Q>, LU_LDS_LIMIT));
     for (int p0 = 1; p0 <= t.dn; p0 += LU_NB) {
       hipLaunchKernelGGL(k_lu_panel<Q>, dim3(1), dim3(LU_NB * 64), 0, c.stream, c.dAB, c.dipiv, c.dju, c.d_lustate,
                          t.dn, t.dkl, t.dku, p0);

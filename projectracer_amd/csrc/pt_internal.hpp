@@ -17,6 +17,7 @@
 #include <string>
 #include <vector>
 #include "../../include/projectracer_gpu.h"
+#include "pt_once.hpp"
 
 namespace pt {
 
@@ -233,6 +234,15 @@ void set_error(const std::string& s);
     int rc_ = (call);             \
     if (rc_ != PT_OK) return rc_; \
   } while (0)
+
+// kernel KERN may ask for BYTES of dynamic LDS on the context's device
+template <class K>
+int allow_lds(Context& c, OncePerDevice& once, K* kern, size_t bytes) {
+  PT_HIP(static_cast<hipError_t>(once.apply(c.device, [&] {
+    return (int)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+  })));
+  return PT_OK;
+}
 
 // ---- solver (pt_solver.hip) ------------------------------------------------
 int solver_alloc(Context& c);

@@ -1457,10 +1457,8 @@ static SweepArgs<R> sweep_args(Context& c, int l, bool f32, const LevelRkc& rk, 
 template <typename R, int EV, int RB, bool PW2>
 static int launch_sweep_t(Context& c, const SweepShape& s, const SweepArgs<R>& a) {
   constexpr int NT = sweep_threads<R, EV, RB>();
-  // set once per process (a thread-safe static initialisation)
-  static const hipError_t attr_rc = hipFuncSetAttribute((const void*)k_sweep<R, EV, RB, NT, PW2>,
-                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)SWEEP_LDS_BYTES);
-  PT_HIP(attr_rc);
+  static OncePerDevice lds;
+  PT_TRY(allow_lds(c, lds, k_sweep<R, EV, RB, NT, PW2>, SWEEP_LDS_BYTES));
   hipLaunchKernelGGL((k_sweep<R, EV, RB, NT, PW2>), dim3(s.nblk), dim3(s.threads), s.lds, c.stream, a);
   return PT_OK;
 }
@@ -1536,10 +1534,8 @@ static int sweep_level(Context& c, int l, bool f32, const LevelRkc& rk, double c
 }
 
 static int launch_coarse_apply_wg(Context& c, const float* rhs, float* err, int n, int m, int pitch, float sz) {
-  // set once per process (a thread-safe static initialisation)
-  static const hipError_t attr_rc = hipFuncSetAttribute((const void*)k_coarse_apply_wg, hipFuncAttributeMaxDynamicSharedMemorySize,
-                               (int)SMALL_LDS_BYTES);
-  PT_HIP(attr_rc);
+  static OncePerDevice limit;
+  PT_TRY(allow_lds(c, limit, k_coarse_apply_wg, SMALL_LDS_BYTES));
   const size_t lds = sizeof(double) * (1 + CA_SEG) * c.nci;
   if (lds > SMALL_LDS_BYTES) {
     set_error("coarsest grid too large for the single-workgroup coarse operator");

@@ -1122,10 +1122,8 @@ static FilterArgs filter_args(const Context& c, bool comp) {
 }
 template <bool COMP, bool PW2>
 static int launch_filter(Context& c, const FilterArgs& a, const FilterLaunch& f, int threads, size_t lds) {
-  // set once per process (a thread-safe static initialisation)
-  static const hipError_t attr_rc = hipFuncSetAttribute((const void*)k_filter_passes<COMP, PW2>,
-                               hipFuncAttributeMaxDynamicSharedMemorySize, FILTER_LDS_BYTES);
-  PT_HIP(attr_rc);
+  static OncePerDevice limit;
+  PT_TRY(allow_lds(c, limit, k_filter_passes<COMP, PW2>, FILTER_LDS_BYTES));
   hipLaunchKernelGGL((k_filter_passes<COMP, PW2>), dim3(a.ntile), dim3(threads), lds, c.stream, a, f);
   return PT_OK;
 }
