@@ -162,6 +162,8 @@ int pt_create(const pt_params* p, void** out) {
   c->filter_on_device = !(filter_env && filter_env[0] == '1');
   const char* radix_env = std::getenv("PT_PROJECT_RADIX");
   c->project_radix_only = radix_env && radix_env[0] == '1';
+  const char* sweep_env = std::getenv("PT_SWEEP_STAGES");
+  if (sweep_env) c->sweep_stages = std::max(0, std::atoi(sweep_env));
   int rc = build_tables(c->P, c->T);
   if (rc != PT_OK) { delete c; return rc; }
   c->P.nx = c->T.nx; c->P.nz = c->T.nz; c->P.grids = c->T.grids;

@@ -191,6 +191,7 @@ struct Context {
   int cyc[52] = {0};
   int cyc_n = 0;
   bool coarse_zero = false;
+  int sweep_stages = 0;      // most stages per launch of a sweep (PT_SWEEP_STAGES at pt_create; 0: as the plan takes)
   int presmooth_from = 99;   // the mixed path's cycle smooths levels >= this on the way up only (2 by default)
   std::vector<CycleGraph> cycle_graphs;
   // mixed precision work

@@ -1402,6 +1402,7 @@ static SweepPlan sweep_plan(const Context& c, int l, bool f32, int s) {
         if (cw > n - 1 || ch > m - 1) continue;
         for (int ns = 1; ns <= s; ns++) {
           const int nseg = (s + ns - 1) / ns, base = s / nseg, rem = s % nseg;
+          if (c.sweep_stages > 0 && ns > c.sweep_stages) break;
           if (base + (rem ? 1 : 0) != ns) continue;   // a larger ns with as many launches
           const SweepShape widest = sweep_shape(n, m, cw, ch, rb, ns + extra, elem);
           if (widest.threads > sweep_threads_of(f32, ev, rb) || widest.lds > SWEEP_LDS_BYTES) break;
