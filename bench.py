@@ -42,21 +42,28 @@ ROOT = Path(__file__).resolve().parent
 sys.path.insert(0, str(ROOT))
 
 HBM_PEAK_GBS = 8000.0
-# Algorithmic bytes of one RKC1 stage per interior point with the general
-# (variable-viscosity) operator: read S1 (the stencil source, once), S0, S2,
-# eta, eta_xx-eta_zz, eta_xz, eta_x, eta_z, RHS, dt_stream and write Y: 11
-# words.  FP32 (the mixed path's smoother) 44 B, FP64 88 B.  The isoviscous
-# operator reads 4 words fewer.
-STAGE_WORDS = {"general": 11, "isoviscous": 7}
+# FP32 vector peak without packed instructions (the library is built without
+# them): 256 CUs x 4 SIMDs x 16 lanes x 2 FLOP per FMA x 2.4 GHz.
+FP32_PEAK_TFLOPS = 78.6
+# Operations of one RKC1 stage per interior point (FP32, an FMA counted as
+# two).  General operator: 117 weighted sums' FMAs, 29 for the products and
+# sums of stream_space, 8 for the stage update.  Isoviscous: 39 FMAs, 8 and 8.
+STAGE_FLOPS = {"general": 271, "isoviscous": 94}
+# Words a sweep cannot do without per interior point, however many launches it
+# takes: read psi, eta, eta_xx-eta_zz, eta_xz, eta_x, eta_z, RHS, dt_stream and
+# write psi: 9 words (36 B in FP32).  The isoviscous operator reads 4 fewer.
+SWEEP_WORDS = {"general": 9, "isoviscous": 5}
+# RKC1 stages per sweep of the mixed path: level 1 and the levels below
+SWEEP_STAGES = {"stage_l1": 35, "stage_coarse": 15}
 # Tracer pipeline per tracer and step: the four RK4 stage kernels move
 # 96+112+112+88 B; each of the five projections reads r, s, T, C (32 B).
 RK_BYTES_PER_TRACER_STEP = 408
 RK2_BYTES_PER_TRACER = 112
 PROJECT_BYTES_PER_TRACER = 32
 PROJECTIONS_PER_STEP = 5
-# One filter pass over the node field (halo included) reads the field once
-# and writes it once; its check reads it once: 24 B per node.
-FILTER_BYTES_PER_NODE = 24
+# A filter loop, however many passes it makes, reads its node field (halo
+# included) once and writes it once.
+FILTER_BYTES_PER_NODE = 16
 
 # Viscosity laws of the 1024x256 workload (see the module docstring).
 WORKLOADS = {
@@ -427,46 +434,59 @@ def cpu_baseline(args):
                 seconds_per_step=sec, tracer_updates_per_s=case.ntr / sec)
 
 
-def stage_roofline(ev, words, bytes_per_word, label):
+# HBM bytes per launch of the mixed path's FP32 sweep kernel, measured with
+# rocprofv3 FETCH_SIZE / WRITE_SIZE on the 1024x256 law and calibrated on a
+# known copy (the tables they come from are in cases_kernel_stats.md beside it)
+SWEEP_TRAFFIC = ROOT / "profiles" / "k_sweep_f32_general_1024x256_traffic.json"
+
+
+def sweep_traffic(args, ev):
+    """Measured HBM bytes per sweep launch, weighted by this run's launch mix
+    (level 1 against the levels below); None off the profiled workload."""
+    if args.workload != "law" or (args.nx, args.nz) != (1024, 256) or not SWEEP_TRAFFIC.exists():
+        return None
+    t = json.loads(SWEEP_TRAFFIC.read_text())
+    l1, co = ev["stage_l1"]["launches"], ev["stage_coarse"]["launches"]
+    if l1 + co == 0:
+        return None
+    return (l1 * t["level1_bytes_per_launch"] + co * t["coarse_bytes_per_launch"]) / (l1 + co)
+
+
+def sweep_roofline(ev, flops, label):
     """Roofline of the RKC1 sweep kernel from the event steps: all its
-    launches, the algorithmic bytes of each being its interior points times
-    its stages times a stage's words."""
+    launches, each doing its interior points times its stages times a stage's
+    operations (the overlap that neighbouring tiles both compute not counted)."""
     l1, co = ev["stage_l1"], ev["stage_coarse"]
     ms = l1["ms"] + co["ms"]
     n = l1["launches"] + co["launches"]
-    bpp = words * bytes_per_word
-    total_bytes = bpp * (l1["work"] + co["work"])
     if n == 0 or ms <= 0:
         return None
-    avg_us = 1e3 * ms / n
-    achieved = total_bytes / n / (avg_us * 1e-6) / 1e9
-    l1_us = 1e3 * l1["ms"] / max(1, l1["launches"])
-    co_us = 1e3 * co["ms"] / max(1, co["launches"])
+
+    def part(x):
+        us = 1e3 * x["ms"] / max(1, x["launches"])
+        return {"launches": x["launches"], "avg_launch_us": us,
+                "point_stages_per_launch": x["work"] / max(1, x["launches"]),
+                "achieved_TFLOPS": flops * x["work"] / (x["ms"] * 1e-3) / 1e12 if x["ms"] > 0 else None}
+
+    achieved = flops * (l1["work"] + co["work"]) / (ms * 1e-3) / 1e12
     return {
-        "kernel": label, "bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
-        "frac": achieved / HBM_PEAK_GBS, "traffic": None,
-        "avg_launch_us": avg_us, "launches": n, "bytes_per_launch": total_bytes / n,
-        "bytes_per_point": bpp, "ms_per_step": ms / ev["steps"],
-        "level1": {"launches": l1["launches"], "avg_launch_us": l1_us,
-                   "bytes_per_launch": bpp * l1["work"] / max(1, l1["launches"]),
-                   "achieved_GBs": bpp * l1["work"] / max(1, l1["launches"]) / (l1_us * 1e-6) / 1e9},
-        "coarse_levels": {"launches": co["launches"], "avg_launch_us": co_us,
-                          "bytes_per_launch": bpp * co["work"] / max(1, co["launches"]),
-                          "achieved_GBs": bpp * co["work"] / max(1, co["launches"]) / (co_us * 1e-6) / 1e9
-                          if co["launches"] else None},
+        "kernel": label, "bound": "fp32 vector", "achieved": achieved, "peak": FP32_PEAK_TFLOPS, "unit": "TFLOP/s",
+        "frac": achieved / FP32_PEAK_TFLOPS, "traffic": None,
+        "avg_launch_us": 1e3 * ms / n, "launches": n, "flops_per_point_stage": flops, "ms_per_step": ms / ev["steps"],
+        "level1": part(l1), "coarse_levels": part(co),
     }
 
 
 def step_bytes(ev, r, words, bytes_per_word):
-    """Algorithmic bytes of one step: every stage launch's points x words,
-    the tracer pipeline, and the filter passes of the last projection
-    (n_comp, plus the first nine C passes when it is nonzero, and n_temp)
-    over the halo-3 node field, for each of the five projections."""
-    solver = words * bytes_per_word * (ev["stage_l1"]["work"] + ev["stage_coarse"]["work"]) / ev["steps"]
+    """Bytes one step cannot do without: every sweep's operands and result
+    once, the tracer pipeline, and each filter loop's field in and out once,
+    for each of the five projections."""
+    sweeps = sum(ev[k]["work"] / stages for k, stages in SWEEP_STAGES.items())   # interior points, once per sweep
+    solver = words * bytes_per_word * sweeps / ev["steps"]
     tracers = (RK_BYTES_PER_TRACER_STEP + PROJECTIONS_PER_STEP * PROJECT_BYTES_PER_TRACER) * r["ntr"]
     nodes = (r["nx"] + 7) * (r["nz"] + 7)
-    passes = r["n_comp"] + 9 * (r["n_comp"] > 0) + r["n_temp"]
-    filters = PROJECTIONS_PER_STEP * passes * FILTER_BYTES_PER_NODE * nodes
+    loops = (r["n_comp"] > 0) + (r["n_temp"] > 0)
+    filters = PROJECTIONS_PER_STEP * loops * FILTER_BYTES_PER_NODE * nodes
     return solver + tracers + filters, dict(solver=solver, tracers=tracers, filters=filters)
 
 
@@ -516,12 +536,15 @@ def main():
     den = float(np.max(np.abs(fp64["sf_first"])))
     mixed_err = float(np.max(np.abs(mixed["sf_first"] - fp64["sf_first"]))) / den
     general = args.workload != "isoviscous"
-    words = STAGE_WORDS["general" if general else "isoviscous"]
+    form = "general" if general else "isoviscous"
     ev = mixed["events"]
-    roof = stage_roofline(ev, words, 4, "k_sweep<float, %s> (RKC1 sweeps of the mixed path's FP32 V-cycle, several "
-                          "stages per launch; bytes counted per stage)"
-                          % ("general operator" if general else "isoviscous"))
-    sb, sb_parts = step_bytes(ev, mixed, words, 4)
+    roof = sweep_roofline(ev, STAGE_FLOPS[form], "k_sweep<float, %s> (RKC1 sweeps of the mixed path's FP32 V-cycle, "
+                          "several stages per launch)" % ("general operator" if general else "isoviscous"))
+    if roof is not None:
+        roof["traffic"] = sweep_traffic(args, ev)
+        if roof["traffic"] is not None:
+            roof["traffic_source"] = str(SWEEP_TRAFFIC.relative_to(ROOT))
+    sb, sb_parts = step_bytes(ev, mixed, SWEEP_WORDS[form], 4)
     ntr = mixed["ntr"]
     rk_ms_step = ev["tracer_stages"]["ms"] / ev["steps"]
     rk2_us = 1e3 * ev["rk2"]["ms"] / max(1, ev["rk2"]["launches"])
