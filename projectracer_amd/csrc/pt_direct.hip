@@ -170,8 +170,8 @@ __global__ void k_sf_assemble(SfArgs a, const double* vis, double* ab) {
 // are first written by the step that DGBTF2 zeroes them at, so that zeroing
 // is not repeated.
 // Bound by the chain of steps: apply to the next column, pivot search, scaling,
-// barrier, one compute unit at work.  100x100 (n = 10201, kl = 303), build in
-// all: 38.6 ms with a thread per row, the panel in LDS and three barriers per
+// barrier, one compute unit at work.  100x100 (n = 10201, kl = 303), device
+// time of the build: 38.6 ms with a thread per row, the panel in LDS and three barriers per
 // column (panel of 32: 100 us; trailing columns in LDS 25 us); 14.5 ms now
 // (panel of 16: 14.2 us, trailing 8.0 us).  With rows per thread and the panel
 // in registers every column's pivot row passes through LDS, in any form of it
@@ -425,7 +425,7 @@ __global__ void __launch_bounds__(LU_TRAIL_WAVES * 64) k_lu_trailing(double* ab,
 //     is zero, then b(j-1 .. j-kl-ku) -= x(j) U(., j).
 // Bound by the chain of a block (head 1.7 us forward, 3.5 us backward with its
 // quotients; then the tail) and by what one compute unit draws from memory,
-// about 40 GB/s.  At 100x100 (160 blocks, bands 303 and 606) forward and
+// 40 GB/s (31 and 56 MB a solve, by counters).  At 100x100 (160 blocks, bands 303 and 606) forward and
 // backward took 1.73 and 3.56 ms with the loads between the barriers, masked
 // steps and divisions, and take 0.78 and 1.39 ms.  (Reloading each register
 // right after its step would use the tail's time too, but the compiler gives

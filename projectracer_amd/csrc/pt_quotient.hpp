@@ -8,7 +8,9 @@ namespace pt {
 // s / d, correctly rounded, from rd = RN(1/d).  PW2: d is a power of two and
 // the product is the quotient.  Otherwise two residual corrections: the first
 // leaves q within one unit of the quotient, and then the second rounds it
-// correctly (Markstein's theorem).  A quotient that overflows is returned as
+// correctly (Markstein's theorem), as long as the residuals are representable:
+// from |s| = 2^-969 on.  Below, their low bits underflow and the quotient may be
+// one unit in the last place off.  A quotient that overflows is returned as
 // it is (the correction of an infinity would be NaN).  5 (1) instructions
 // against about 14 of the hardware's division sequence.
 template <bool PW2>

@@ -283,6 +283,12 @@ constexpr int SMALL_THREADS = 1024;
 // operations and their order are those of one stage per launch
 // (stream_space_pt, or the factorised form below), so the results do not
 // depend on the tiling.
+// Bound by the issue of vector instructions, the overlap's among them, and by
+// what a launch costs around them (window, barriers, start and end).  1024x256,
+// general operator, FP32, by counters: level 1 (256 tiles, 3 stages) 13.6 us with
+// 57% of the issue slots taken, LDS active 18%, 27 MB from and to HBM (its
+// operands once: 12.5); levels 2 to 5 8.5, 6.5, 6.2 and 8.2 us with 37, 28, 24
+// and 40% on the compute units they use.  FP64 isoviscous, level 1: 13.6 us, 42%.
 // ---------------------------------------------------------------------------
 constexpr int SWEEP_MAX_STAGES = 64;
 
@@ -1331,9 +1337,13 @@ static SweepShape sweep_shape(int n, int m, int cw, int ch, int rb, int nev, siz
   return s;
 }
 
-// the operator's form on a level: general, isoviscous, or (FP32 levels >= 2
-// that one workgroup or column strips of at most 64 rows cover) isoviscous
-// with the factorised psi_xxzz
+// the operator's form on a level: general (0), isoviscous (1), or isoviscous
+// with the factorised psi_xxzz (2), on some of the FP32 levels >= 2.  k_sweep
+// takes either on any level, and both are right to FP32 rounding.  The limits
+// below are those of the kernels that these levels had before k_sweep; they are
+// kept for one reason: the form decides the rounding of the FP32 corrections,
+// so with other limits a mixed solve of the same input would end at another psi
+// within its stop test's tolerance.
 static int sweep_form(const Context& c, int l, bool f32) {
   if (c.P.ivis != 0) return 0;
   if (!f32 || l < 2) return 1;
@@ -1345,10 +1355,8 @@ static int sweep_form(const Context& c, int l, bool f32) {
   return (b4 <= SMALL_THREADS && 2 * b4 >= SMALL_THREADS) || npts <= SMALL_THREADS ? 2 : 1;
 }
 
-// Modelled time (us) of one launch of `nev` evaluations; the model's terms
-// and the constants per operator form are a fit to 14,000 measured sweeps of
-// 30 levels from 7x7 to 1023x255 points (its choice is within 2% of the
-// measured best on 28 of them, within 9% on all):
+// Modelled time (us) of one launch of `nev` evaluations; the constants per
+// operator form are a fit to timed sweeps of levels from 7x7 to 1023x255 points:
 //   2.9            launch to launch
 //   fill, row      window loads per thread and per window row
 //   stage          an evaluation's latency (LDS round trip, barrier)
@@ -1380,7 +1388,13 @@ static double sweep_launch_us(const SweepCost& k, int n, int m, int cw, int ch, 
 // isoviscous 144 us against 35 x 6.0); 256x64: 16x4, 3, 1 (FP32 general, 15
 // stages: 30 us against 15 x 5.5); 32x32 FP64: one workgroup, all stages, 2
 // points per thread (49 us; one point per thread and a row of LDS reads per
-// point: 58).
+// point: 58).  Whole solves with the stages per launch bounded at 1, 2, 3, 4, 5,
+// 6 and 8 (tile and rows as the model then takes them) and as the plan is, ms:
+//   1024x256 law, mixed    16.6  13.1  11.8  11.7  11.6  11.6  11.6   11.7
+//   1024x256 iso, mixed     9.1   6.7   5.7   5.7   5.5   5.5   5.7    5.5
+//   1024x256 iso, FP64     50.4  31.8  26.1  25.0  24.1  24.1  24.2   23.1
+//   256x64 law, FP64       47.8  29.1  24.2  22.0  21.1  20.3  20.0   18.0
+//   64x64 law, FP64        42.4  27.1  22.2  19.7  18.6  17.8  17.3   14.7
 static SweepPlan sweep_plan(const Context& c, int l, bool f32, int s) {
   const LevelGeom& g = c.L[l].g;
   const int n = g.n, m = g.m, ev = sweep_form(c, l, f32);
@@ -1407,8 +1421,8 @@ static SweepPlan sweep_plan(const Context& c, int l, bool f32, int s) {
           const SweepShape widest = sweep_shape(n, m, cw, ch, rb, ns + extra, elem);
           if (widest.threads > sweep_threads_of(f32, ev, rb) || widest.lds > SWEEP_LDS_BYTES) break;
           // not the tilings whose tiles mostly recompute each other's points, nor
-          // those of several points per thread in few wavefronts: the model does
-          // not hold there
+          // those of several points per thread in few wavefronts: the model was
+          // not fitted to such and calls some of them fast that are not
           double evals = 0.0;
           for (int h = 0; h < ns; h++) evals += (double)std::min(cw + 6 * h, n - 1) * std::min(ch + 6 * h, m - 1);
           if (widest.nblk > 1 && evals * widest.nblk > (nseg == 1 ? 2.0 : 5.0) * ns * (n - 1) * (m - 1)) continue;
@@ -1595,8 +1609,8 @@ static int iterate_stream_t(Context& c, int l, int p, bool fp32, bool l1_sum) {
   }
   const LevelRkc rk = level_rkc(c, l, fp32);
   // the residual of levels >= 2 comes out of the sweep's last launch; level
-  // 1's carries the L1 sum, and the residual of strip-covered isoviscous
-  // FP32 levels is the unfactorised form's
+  // 1's carries the L1 sum, and that of the larger levels in the factorised form
+  // is the unfactorised form's (a matter of its rounding, as in sweep_form)
   const bool fuse = want_res && l >= 2 && !(sweep_form(c, l, fp32) == 2 && (g.n - 1) * (g.m - 1) > 4096);
   R* res = fp32 ? (R*)L.fres : (R*)L.res;
   for (int it = 1; it <= c.P.Nmulti; it++) {

@@ -614,9 +614,9 @@ static void filter_pass(Context& c, const double* T0, double* out, int h, double
 //
 // One pass per launch (latency-bound: a launch to launch gap, a round trip
 // to memory for the field and one for the previous check) took 5.6 us and 1.5
-// us of gap at 1024x256.  Eight passes per launch, bound by the FP64 units and
-// LDS of the CUs (2.4 times the nodes for the overlap) and by 8 us per launch,
-// take 2.9 us each.
+// us of gap at 1024x256.  Eight passes per launch take 2.9 us each: 20.3 us a
+// launch, of which vector instructions take 50% of the issue slots and LDS is
+// active 41% (by counters; 2.4 times the nodes for the overlap), and the gap.
 // ---------------------------------------------------------------------------
 constexpr int FILTER_KMAX = 8;      // passes per launch
 constexpr int FILTER_RB = 5;        // nodes per thread, vertically adjacent
